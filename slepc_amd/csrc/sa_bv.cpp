@@ -39,7 +39,7 @@ static int bv_alloc_impl(BV &V, int64_t n, int m, int prec) {
   SA_HIP(hipMemsetAsync(V.dbuf, 0, sizeof(double) * (size_t)m * m, stream()));
   SA_HIP(hipMalloc(&V.st, sizeof(GsState) * GS_NSTATE));
   SA_HIP(hipMemsetAsync(V.st, 0, sizeof(GsState) * GS_NSTATE, stream()));
-  SA_HIP(hipHostMalloc((void **)&V.st_host, sizeof(GsState)));
+  SA_HIP(hipHostMalloc((void **)&V.st_host, sizeof(GsMirror)));
   // Partition rows into workgroup ranges of whole 64-row chunks.
   const int64_t chunks = std::max<int64_t>(1, (n + 63) / 64);
   // at most gs_max_blocks() workgroups (1024, or 4096 for a basis larger than
@@ -59,6 +59,11 @@ static int bv_alloc_impl(BV &V, int64_t n, int m, int prec) {
   // the reductions read every partial row even after a slot that produced none
   SA_HIP(hipMemsetAsync(V.ws.part, 0, sizeof(double) * 2 * (size_t)G * (GS_MAXC + 1), stream()));
   SA_HIP(hipMemsetAsync(V.ws.dots, 0, sizeof(double) * 2 * (GS_MAXC + 1), stream()));
+  V.ps.bytes = ps_bytes(n, prec);
+  if (V.ps.bytes) {
+    SA_HIP(hipMalloc(&V.ps.words, V.ps.bytes));
+    SA_HIP(hipMemsetAsync(V.ps.words, 0, V.ps.bytes, stream()));
+  }
   SA_HIP(hipMalloc(&V.dq, sizeof(double) * (size_t)m * m + 64 * sizeof(double)));
   SA_HIP(hipHostMalloc((void **)&V.hq, sizeof(double) * (size_t)m * m + 64 * sizeof(double)));
   SA_HIP(hipStreamSynchronize(stream()));
@@ -72,6 +77,7 @@ void bv_free(BV &V) {
   if (V.st_host) (void)hipHostFree(V.st_host);
   if (V.ws.part) (void)hipFree(V.ws.part);
   if (V.ws.dots) (void)hipFree(V.ws.dots);
+  if (V.ps.words) (void)hipFree(V.ps.words);
   if (V.dq) (void)hipFree(V.dq);
   if (V.hq) (void)hipHostFree(V.hq);
   V = BV();
@@ -88,10 +94,14 @@ int bv_sweep(BV &V, const Mat &A, int k, int *m, double eta, double *beta, int *
   SA_CHECK(k >= 0 && *m > k && *m < V.m, "invalid Arnoldi range");
   SA_CHECK(A.prec == V.prec && A.n == V.n, "matrix and basis sizes or precisions differ");
   hipStream_t s = stream();
-  SA_TRY(launch_gs_reset(V, s));
-  for (int j = k; j < *m; j++) SA_TRY(launch_gs_column(V, &A, j + 1, eta, s));
-  SA_HIP(hipMemcpyAsync(V.st_host, V.st + 2, sizeof(GsState), hipMemcpyDeviceToHost, s));
-  SA_HIP(hipStreamSynchronize(s));
+  bool resident = false;
+  SA_TRY(ps_sweep(V, &A, k + 1, *m, eta, s, &resident));
+  if (!resident) {
+    SA_TRY(launch_gs_reset(V, s));
+    for (int j = k; j < *m; j++) SA_TRY(launch_gs_column(V, &A, j + 1, eta, s));
+    SA_HIP(hipMemcpyAsync(V.st_host, V.st + 2, sizeof(GsState), hipMemcpyDeviceToHost, s));
+    SA_HIP(hipStreamSynchronize(s));
+  }
   const GsState &st = *V.st_host;
   if (st.stop) {
     *m = st.stop_col;
@@ -197,10 +207,14 @@ int bv_sweep_deflated(BV &V, const Mat &A, KspWork *w, double rtol, int max_it, 
 // BVOrthonormalizeColumn(V,j,PETSC_FALSE,&norm,&lindep) (bvorthog.c:380-427)
 int bv_orthonormalize(BV &V, int j, double eta, double *norm, int *lindep) {
   hipStream_t s = stream();
-  SA_TRY(launch_gs_reset(V, s));
-  SA_TRY(launch_gs_column(V, nullptr, j, eta, s));
-  SA_HIP(hipMemcpyAsync(V.st_host, V.st + 2, sizeof(GsState), hipMemcpyDeviceToHost, s));
-  SA_HIP(hipStreamSynchronize(s));
+  bool resident = false;
+  SA_TRY(ps_sweep(V, nullptr, j, j, eta, s, &resident));
+  if (!resident) {
+    SA_TRY(launch_gs_reset(V, s));
+    SA_TRY(launch_gs_column(V, nullptr, j, eta, s));
+    SA_HIP(hipMemcpyAsync(V.st_host, V.st + 2, sizeof(GsState), hipMemcpyDeviceToHost, s));
+    SA_HIP(hipStreamSynchronize(s));
+  }
   if (norm) *norm = V.st_host->nrm;
   if (lindep) *lindep = V.st_host->lindep;
   V.passes_done = V.st_host->passes_total;

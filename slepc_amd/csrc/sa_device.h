@@ -2,6 +2,7 @@
 // wave size 64, 256-thread workgroups).
 #pragma once
 #include <hip/hip_runtime.h>
+#include <cstdint>
 
 namespace sa {
 
@@ -31,6 +32,94 @@ constexpr int N_XCD = 8;
 __device__ __forceinline__ int xcd_block(int b, int G) {
   const int q = G / N_XCD, r = G % N_XCD, x = b % N_XCD, i = b / N_XCD;
   return x * q + min(x, r) + i;
+}
+
+// Cross-lane sums of a wave in the vector ALU (DPP within rows of 16 lanes,
+// the gfx950 row and half swaps beyond them): a few cycles per step, where
+// a shuffle through the LDS unit costs over a hundred.
+template <int CTRL>
+__device__ __forceinline__ double dpp_mov(double v) {
+  const uint64_t u = __builtin_bit_cast(uint64_t, v);
+  const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, CTRL, 0xf, 0xf, true);
+  const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), CTRL, 0xf, 0xf, true);
+  return __builtin_bit_cast(double, ((uint64_t)hi << 32) | lo);
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_mov(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, true));
+}
+constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E;             // quad_perm [1,0,3,2], [2,3,0,1]
+constexpr int DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140;  // lane ^ 7 in 8 lanes, lane ^ 15 in 16
+constexpr int DPP_ROR8 = 0x128;                             // lane ^ 8 in 16 lanes
+
+// Lanes below M of each 2M lanes return x + (x of lane + M), the others
+// y + (y of lane - M), M = 32 or 16: one step of a reduce-scatter, and with
+// y = x the sum over the pair.
+template <int M>
+__device__ __forceinline__ uint32_t swap_lanes(uint32_t x, uint32_t y, uint32_t *other) {
+  static_assert(M == 32 || M == 16, "rows of 16 lanes or halves of the wave");
+  if constexpr (M == 32) {
+    const auto r = __builtin_amdgcn_permlane32_swap(x, y, false, false);
+    *other = r[1];
+    return r[0];
+  } else {
+    const auto r = __builtin_amdgcn_permlane16_swap(x, y, false, false);
+    *other = r[1];
+    return r[0];
+  }
+}
+template <int M>
+__device__ __forceinline__ double swap_add(double x, double y) {
+  const uint64_t a = __builtin_bit_cast(uint64_t, x), b = __builtin_bit_cast(uint64_t, y);
+  uint32_t lo1, hi1;
+  const uint32_t lo0 = swap_lanes<M>((uint32_t)a, (uint32_t)b, &lo1);
+  const uint32_t hi0 = swap_lanes<M>((uint32_t)(a >> 32), (uint32_t)(b >> 32), &hi1);
+  return __builtin_bit_cast(double, ((uint64_t)hi0 << 32) | lo0) +
+         __builtin_bit_cast(double, ((uint64_t)hi1 << 32) | lo1);
+}
+template <int M>
+__device__ __forceinline__ float swap_add(float x, float y) {
+  uint32_t o;
+  const uint32_t k = swap_lanes<M>(__builtin_bit_cast(uint32_t, x), __builtin_bit_cast(uint32_t, y), &o);
+  return __builtin_bit_cast(float, k) + __builtin_bit_cast(float, o);
+}
+// The sum over N consecutive lanes (a power of two), in each of them.
+template <int N, typename T>
+__device__ __forceinline__ T lanes_sum(T v) {
+  if constexpr (N >= 2) v += dpp_mov<DPP_XOR1>(v);
+  if constexpr (N >= 4) v += dpp_mov<DPP_XOR2>(v);
+  if constexpr (N >= 8) v += dpp_mov<DPP_HALF_MIRROR>(v);
+  if constexpr (N >= 16) v += dpp_mov<DPP_MIRROR>(v);
+  if constexpr (N >= 32) v = swap_add<16>(v, v);
+  if constexpr (N >= 64) v = swap_add<32>(v, v);
+  return v;
+}
+// One step of a reduce-scatter at lane bit M: lanes with the bit clear keep x,
+// the others y, and add their partner's copy of it.
+template <int M, typename T>
+__device__ __forceinline__ T scatter_add(T x, T y, int lane) {
+  if constexpr (M >= 16) {
+    return swap_add<M>(x, y);
+  } else {
+    constexpr int CTRL = M == 8 ? DPP_ROR8 : (M == 4 ? DPP_HALF_MIRROR : (M == 2 ? DPP_XOR2 : DPP_XOR1));
+    const bool hi = (lane & M) != 0;
+    asm volatile("" : "+v"(x), "+v"(y));   // keeps the choice a select, not an indexed read
+    return (hi ? y : x) + dpp_mov<CTRL>(hi ? x : y);
+  }
+}
+// Reduce-scatter of p[0..N) over the wave (N a power of two up to 64): lane l
+// returns the sum over the lanes of p[l / (64 / N)].
+template <int N, int M = 32, typename T>
+__device__ __forceinline__ T wave_scatter(T (&p)[N], int lane) {
+  constexpr int H = N * M / 64;            // values each lane keeps after this step
+  if constexpr (H >= 1) {
+#pragma unroll
+    for (int i = 0; i < H; i++) p[i] = scatter_add<M>(p[i], p[i + H], lane);
+    if constexpr (M > 1) return wave_scatter<N, M / 2>(p, lane);
+    else return p[0];
+  } else {
+    return lanes_sum<2 * M>(p[0]);
+  }
 }
 
 // out[col] = sum_b part[col * G + b] for col < ncol.  Each wave reduces four

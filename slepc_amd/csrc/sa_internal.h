@@ -68,10 +68,22 @@ struct GsState {
   double onrm, nrm, beta;
 };
 
+struct GsMirror {   // pinned host memory: the state, and what a resident sweep reports
+  GsState st;
+  int ok;           // its lead workgroup finished
+  int fail;         // one of its workgroups gave up waiting
+};
+
 struct Workspace {           // device scratch for partial sums of one BV
   double *part = nullptr;    // 2 x [GS_MAXC+1][maxG], column-major partial sums
   double *dots = nullptr;    // 2 x [GS_MAXC+1] reduced dot products
   int maxG = 0;
+};
+
+struct PsWork {              // exchange words of the resident sweep (sa_sweep.hip)
+  uint64_t *words = nullptr;
+  size_t bytes = 0;
+  uint32_t tag = 1;          // number of the next exchange
 };
 
 struct BV {
@@ -81,8 +93,9 @@ struct BV {
   void *data = nullptr;        // T[ld * m]
   double *dbuf = nullptr;      // coefficient buffer m x m (FP64) on device
   GsState *st = nullptr;       // device, GS_NSTATE states (ping-pong)
-  GsState *st_host = nullptr;  // pinned host mirror of st[2]
+  GsState *st_host = nullptr;  // pinned host mirror of st[2] (a GsMirror)
   Workspace ws;
+  PsWork ps;
   double *dq = nullptr;        // device staging for Q / q vectors (m*m doubles)
   double *hq = nullptr;        // pinned host staging
   int G = 0, rows_per_block = 0;
@@ -117,6 +130,13 @@ int mat_norm_inf(const Mat &A, double *out);
 int launch_gs_column(BV &V, const Mat *A, int c, double eta, hipStream_t s);
 // Clears the Gram-Schmidt state machine of V before a sweep.
 int launch_gs_reset(BV &V, hipStream_t s);
+// Columns c0..c1 of V by one resident kernel (sa_sweep.hip): with A each is A
+// times the one before it, orthonormalised; without A, c0 = c1 and column c0
+// itself is.  *done is false when the basis does not fit or the kernel gave
+// up (nothing has changed then); else V.st and V.st_host hold the state.
+// Blocks on the stream.
+int ps_sweep(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool *done);
+size_t ps_bytes(int64_t n, int prec);   // bytes of its exchange words, 0 when no basis of n rows fits
 int gs_min_chunks(bool big);   // fewest 64-row chunks per workgroup of the GS kernels (big: above GS_NT_BYTES)
 int concurrent_solves();      // the application's hint (sa_set_concurrent_solves)
 int gs_max_blocks(bool big);  // most workgroups of the GS kernels per basis (big: above GS_NT_BYTES)

@@ -1,0 +1,108 @@
+"""The resident Arnoldi sweep (csrc/sa_sweep.hip): the Arnoldi relation and
+orthogonality at the edges of its row blocks, column slots and operator
+staging, and the same results when its waits give up and the sweep runs slot
+by slot instead."""
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+EPS = {"fp64": 2.2e-16, "fp32": 6e-8}
+
+
+def _csr(sa, kind, n, seed=3):
+    """band: neighbours and a far diagonal; ragged: empty rows and rows whose
+    columns are spread over the whole matrix (more remote entries than the
+    resident kernel lists, so that it reads the operator from memory)."""
+    rng = np.random.default_rng(seed)
+    if kind == "band":
+        offs = [0, 1, -1, 37, -211]
+        r, c = zip(*[(np.arange(n), np.arange(n) + o) for o in offs])
+        r, c = np.concatenate(r), np.concatenate(c)
+    else:
+        k = rng.integers(0, 40, n)
+        r = np.repeat(np.arange(n), k)
+        c = rng.integers(0, n, len(r))
+    keep = (c >= 0) & (c < n)
+    r, c = r[keep], c[keep]
+    key = np.unique(r.astype(np.int64) * n + c)
+    r, c = key // n, key % n
+    rp = np.zeros(n + 1, np.int32)
+    rp[1:] = np.cumsum(np.bincount(r, minlength=n))
+    return sa.CSR(n, rp, c.astype(np.int32), rng.uniform(-1.0, 1.0, len(c)))
+
+
+def _matvec(A, X):
+    p = np.concatenate([np.zeros((1, X.shape[1])), np.cumsum(A.val[:, None] * X[A.col], axis=0)])
+    return p[A.rowptr[1:]] - p[A.rowptr[:-1]]
+
+
+# rows: one and two chunks, the last row block with one row, exactly 64 blocks
+# and one row more (1 -> 2 -> 4 chunks per block), 256 blocks of 4 chunks and
+# one row more (6 chunks); columns: the last of a slot, one more, a full basis
+@pytest.mark.parametrize("n,m,kind,prec", [
+    (64, 7, "band", "fp64"), (65, 33, "band", "fp64"), (257, 32, "ragged", "fp64"), (4096, 64, "band", "fp64"),
+    (4097, 65, "ragged", "fp64"), (8193, 97, "band", "fp64"), (16385, 20, "ragged", "fp32"),
+    (65536, 64, "band", "fp64"), (65537, 12, "band", "fp64"), (98305, 40, "band", "fp32"),
+    (4097, 126, "band", "fp32"), (180224, 10, "band", "fp64")])
+def test_sweep_relation(sa, n, m, kind, prec):
+    P = sa.FP64 if prec == "fp64" else sa.FP32
+    A = _csr(sa, kind, n)
+    if prec == "fp32":
+        A.val = A.val.astype(np.float32).astype(np.float64)
+    M, V = sa.Mat(A, P), sa.BV(n, m + 1, P)
+    V.set_column(0, sa.rand_uniform(5, n))
+    V.orthonormalize_column(0)
+    for k in (0, m // 2):                     # a first sweep, and one from column m // 2
+        mm, beta, bd = V.mat_arnoldi(M, k, m)
+        assert mm == m and not bd
+        X, H = V.get_matrix(m + 1), V.coefficients(1, m + 1)
+        assert beta == pytest.approx(H[m, m - 1], rel=1e-15)
+        H = np.vstack([H, np.zeros((m + 1 - H.shape[0], m))]) if H.shape[0] < m + 1 else H[:m + 1]
+        # each column: at most ~40 products per row, m updates, all of size <= 40 * ||x||_2
+        eps = EPS[prec]
+        rel = _matvec(A, X[:, :m]) - X @ np.triu(H, -1)
+        assert np.linalg.norm(rel, axis=0).max() <= 40 * (m + 40) * eps
+        assert np.abs(X.T @ X - np.eye(m + 1)).max() <= 100 * (m + 1) * eps
+
+
+CODE = """
+import sys, numpy as np
+sys.path.insert(0, %r)
+import slepc_amd as sa
+sa.init(0)
+A = sa.lap2d(70, 61)
+V = sa.BV(A.n, 34)
+V.set_column(0, sa.rand_uniform(5, A.n))
+V.orthonormalize_column(0)
+M = sa.Mat(A)
+V.mat_arnoldi(M, 0, 32)
+V.set_column(33, sa.rand_uniform(6, A.n))
+nrm, lindep = V.orthonormalize_column(33)
+np.savez(sys.argv[1], V=V.get_matrix(34), H=V.coefficients(0, 34), nrm=nrm)
+"""
+
+
+def test_sweep_gives_up_and_starts_over(tmp_path):
+    """With no polls allowed, every wait that is not met at once gives up: the
+    kernel ends, and the host's slot-by-slot sweep returns the same basis (the
+    orthonormalised column included, whose input the kernel may have
+    overwritten), to the rounding of two summation orders."""
+    out = []
+    for polls in (None, "0"):
+        env = dict(os.environ)
+        env.pop("SLEPC_AMD_SWEEP_POLLS", None)
+        if polls is not None:
+            env["SLEPC_AMD_SWEEP_POLLS"] = polls
+        f = str(tmp_path / ("r%s.npz" % polls))
+        subprocess.run([sys.executable, "-c", CODE % ROOT, f], check=True, env=env, timeout=100)
+        out.append(np.load(f))
+    a, b = out
+    assert np.abs(a["V"] - b["V"]).max() <= 1e-12
+    assert np.abs(a["H"] - b["H"]).max() <= 1e-13
+    assert float(a["nrm"]) == pytest.approx(float(b["nrm"]), rel=1e-14)

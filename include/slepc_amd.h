@@ -65,10 +65,9 @@ int sa_mat_create_csr(int n, int64_t nnz, const int32_t *rowptr_host, const int3
  * kernels on small operators. */
 int64_t sa_set_spmv_stream_bytes(int64_t bytes);
 /* Partition hint: the number of solves the application keeps in flight at
- * once on the device (one host thread each).  With 2 or more, bases that fit
- * the last-level cache (<= 256 MiB) created afterwards give each
- * Gram-Schmidt workgroup two 64-row chunks instead of one, so the slot
- * kernels of concurrent solves share the CUs.  Default 1; returns the
+ * once on the device (one host thread each).  With 2 or more, the sweeps of
+ * bases created afterwards that fit the GPU's registers take half its CUs
+ * where half hold them, so that two run side by side.  Default 1; returns the
  * previous value.  No counterpart in the reference (PETSc runs one solve per
  * process); results differ from a solve alone only in the rounding of the
  * reductions. */

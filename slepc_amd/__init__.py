@@ -185,8 +185,8 @@ def set_spmv_stream_bytes(nbytes):
 
 def set_concurrent_solves(nsolves):
     """Partition hint: number of solves kept in flight at once (one host
-    thread each); with 2 or more, cache-resident bases created afterwards use
-    half as many Gram-Schmidt workgroups.  Returns the previous value."""
+    thread each); with 2 or more, the sweeps of bases created afterwards use
+    half the CUs where half hold them.  Returns the previous value."""
     return int(lib().sa_set_concurrent_solves(int(nsolves)))
 
 

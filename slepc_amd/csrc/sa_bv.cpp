@@ -42,24 +42,23 @@ static int bv_alloc_impl(BV &V, int64_t n, int m, int prec) {
   SA_HIP(hipHostMalloc((void **)&V.st_host, sizeof(GsMirror)));
   // Partition rows into workgroup ranges of whole 64-row chunks.
   const int64_t chunks = std::max<int64_t>(1, (n + 63) / 64);
-  // at most gs_max_blocks() workgroups (1024, or 4096 for a basis larger than
-  // the last-level cache, whose slot kernels then fit more workgroups per CU)
-  // and at least gs_min_chunks() chunks each, so the reductions of the
-  // partial sums stay short
-  const bool big = V.ld * m * (int64_t)es > GS_NT_BYTES;   // the slot kernels' NT flag
-  const int64_t maxG = gs_max_blocks(big), minc = gs_min_chunks(big);
-  int64_t G = std::min(maxG, std::max<int64_t>(1, (chunks + minc - 1) / minc));
+  // (BVDotVec: at most 1024 workgroups, 4096 for a basis larger than the
+  // last-level cache)
+  const bool big = V.ld * m * (int64_t)es > GS_NT_BYTES;
+  int64_t G = std::min<int64_t>(big ? 4096 : 1024, chunks);
   const int64_t cpb = (chunks + G - 1) / G;
   G = (chunks + cpb - 1) / cpb;
   V.G = (int)G;
   V.rows_per_block = (int)(cpb * 64);
-  V.ws.maxG = (int)G;
-  SA_HIP(hipMalloc(&V.ws.part, sizeof(double) * 2 * (size_t)G * (GS_MAXC + 1)));
+  V.ws.maxG = std::max((int)G, gw_blocks(n, prec, 0));
+  const size_t npart = 2 * (size_t)V.ws.maxG * (GS_MAXC + 1);
+  SA_HIP(hipMalloc(&V.ws.part, sizeof(double) * npart));
   SA_HIP(hipMalloc(&V.ws.dots, sizeof(double) * 2 * (GS_MAXC + 1)));
   // the reductions read every partial row even after a slot that produced none
-  SA_HIP(hipMemsetAsync(V.ws.part, 0, sizeof(double) * 2 * (size_t)G * (GS_MAXC + 1), stream()));
+  SA_HIP(hipMemsetAsync(V.ws.part, 0, sizeof(double) * npart, stream()));
   SA_HIP(hipMemsetAsync(V.ws.dots, 0, sizeof(double) * 2 * (GS_MAXC + 1), stream()));
   V.ps.bytes = ps_bytes(n, prec);
+  V.ps.share = concurrent_solves();
   if (V.ps.bytes) {
     SA_HIP(hipMalloc(&V.ps.words, V.ps.bytes));
     SA_HIP(hipMemsetAsync(V.ps.words, 0, V.ps.bytes, stream()));

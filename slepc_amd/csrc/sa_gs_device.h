@@ -1,6 +1,8 @@
-// Device code of the fused Gram-Schmidt step (SpMV, classical Gram-Schmidt,
-// DGKS refinement "if needed", normalisation), shared by the single-basis
-// sweep (sa_gs.hip) and the lock-step batched sweep (sa_batched.hip).
+// Device code of the Gram-Schmidt step (classical Gram-Schmidt, DGKS refinement
+// "if needed", normalisation): the rule and its states, shared by the resident
+// sweep (sa_sweep.hip), the slots of one basis (sa_gw.hip) and the lock-step
+// batched sweep (sa_batched.hip), and the batched sweep's slots, which fuse the
+// SpMV into slot 1.
 //
 // A column c is orthogonalised by three kernels ("slots"):
 //   slot 1: v = A V(:,c-1) (when a matrix is given) or v = V(:,c); partial
@@ -42,6 +44,11 @@ struct GsArgs {
   double eta;
   int refine;               // BVSetOrthogonalization refinement: GS_REFINE_*
 };
+
+// The slots of one basis (sa_gw.hip): one slot over a.G <= gw_blocks(n, prec, c)
+// workgroups.
+int launch_gw_slot(const GsArgs<double> &a, bool nt, hipStream_t s);
+int launch_gw_slot(const GsArgs<float> &a, bool nt, hipStream_t s);
 
 // The rule of BVOrthogonalizeGS (bvorthog.c:145-217) applied to the dots of
 // one pass: dots[0:c] = V^T v, dots[c] = v^T v, sumsq = sum dots[i]^2.
@@ -104,8 +111,8 @@ __device__ inline int gs_rule(GsState &S, const double *dots, double sumsq, int 
 
 // Thread 0 applies the rule to s_dots; the lead workgroup then records the
 // coefficients (BV_CleanCoefficients + BV_AddCoefficients, bvimpl.h:308-322),
-// the norm at row c and the new state.
-template <typename T>
+// the norm at row c and the new state.  NT: threads of the workgroup.
+template <typename T, int NT = BLK>
 __device__ void gs_decide_block(const GsArgs<T> &a, const double *s_dots, GsState *s_st, int *s_act, int *s_rec,
                                 double *s_scale, bool lead) {
   const int t = threadIdx.x, c = a.c;
@@ -125,7 +132,7 @@ __device__ void gs_decide_block(const GsArgs<T> &a, const double *s_dots, GsStat
     double *h = a.dbuf + (size_t)c * a.m;
     if (*s_rec) {
       const bool first = s_st->pass == 1;
-      for (int i = t; i < c; i += BLK) h[i] = (first ? 0.0 : h[i]) + s_dots[i];
+      for (int i = t; i < c; i += NT) h[i] = (first ? 0.0 : h[i]) + s_dots[i];
     }
     if (t == 0) {
       if (s_st->done) h[c] = s_st->lindep ? 0.0 : s_st->nrm;

@@ -84,6 +84,7 @@ struct PsWork {              // exchange words of the resident sweep (sa_sweep.h
   uint64_t *words = nullptr;
   size_t bytes = 0;
   uint32_t tag = 1;          // number of the next exchange
+  int share = 1;             // sa_set_concurrent_solves when the basis was created
 };
 
 struct BV {
@@ -137,9 +138,8 @@ int launch_gs_reset(BV &V, hipStream_t s);
 // Blocks on the stream.
 int ps_sweep(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool *done);
 size_t ps_bytes(int64_t n, int prec);   // bytes of its exchange words, 0 when no basis of n rows fits
-int gs_min_chunks(bool big);   // fewest 64-row chunks per workgroup of the GS kernels (big: above GS_NT_BYTES)
 int concurrent_solves();      // the application's hint (sa_set_concurrent_solves)
-int gs_max_blocks(bool big);  // most workgroups of the GS kernels per basis (big: above GS_NT_BYTES)
+int gw_blocks(int64_t n, int prec, int c);   // workgroups of a Gram-Schmidt slot of column c (sa_gw.hip)
 int launch_dotvec(BV &V, int l, int k, const void *x, double *q_dev, hipStream_t s);
 int launch_multvec(BV &V, int l, int k, double alpha, const double *q_dev, double beta, void *y,
                    hipStream_t s);

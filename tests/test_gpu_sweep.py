@@ -42,15 +42,7 @@ def _matvec(A, X):
     return p[A.rowptr[1:]] - p[A.rowptr[:-1]]
 
 
-# rows: one and two chunks, the last row block with one row, exactly 64 blocks
-# and one row more (1 -> 2 -> 4 chunks per block), 256 blocks of 4 chunks and
-# one row more (6 chunks); columns: the last of a slot, one more, a full basis
-@pytest.mark.parametrize("n,m,kind,prec", [
-    (64, 7, "band", "fp64"), (65, 33, "band", "fp64"), (257, 32, "ragged", "fp64"), (4096, 64, "band", "fp64"),
-    (4097, 65, "ragged", "fp64"), (8193, 97, "band", "fp64"), (16385, 20, "ragged", "fp32"),
-    (65536, 64, "band", "fp64"), (65537, 12, "band", "fp64"), (98305, 40, "band", "fp32"),
-    (4097, 126, "band", "fp32"), (180224, 10, "band", "fp64")])
-def test_sweep_relation(sa, n, m, kind, prec):
+def check_relation(sa, n, m, kind, prec):
     P = sa.FP64 if prec == "fp64" else sa.FP32
     A = _csr(sa, kind, n)
     if prec == "fp32":
@@ -71,6 +63,18 @@ def test_sweep_relation(sa, n, m, kind, prec):
         assert np.abs(X.T @ X - np.eye(m + 1)).max() <= 100 * (m + 1) * eps
 
 
+# rows: one and two chunks, the last row block with one row, exactly 64 blocks
+# and one row more (1 -> 2 -> 4 chunks per block), 256 blocks of 4 chunks and
+# one row more (6 chunks); columns: the last of a slot, one more, a full basis
+@pytest.mark.parametrize("n,m,kind,prec", [
+    (64, 7, "band", "fp64"), (65, 33, "band", "fp64"), (257, 32, "ragged", "fp64"), (4096, 64, "band", "fp64"),
+    (4097, 65, "ragged", "fp64"), (8193, 97, "band", "fp64"), (16385, 20, "ragged", "fp32"),
+    (65536, 64, "band", "fp64"), (65537, 12, "band", "fp64"), (98305, 40, "band", "fp32"),
+    (4097, 126, "band", "fp32"), (180224, 10, "band", "fp64")])
+def test_sweep_relation(sa, n, m, kind, prec):
+    check_relation(sa, n, m, kind, prec)
+
+
 CODE = """
 import sys, numpy as np
 sys.path.insert(0, %r)
@@ -86,6 +90,40 @@ V.set_column(33, sa.rand_uniform(6, A.n))
 nrm, lindep = V.orthonormalize_column(33)
 np.savez(sys.argv[1], V=V.get_matrix(34), H=V.coefficients(0, 34), nrm=nrm)
 """
+
+
+SLOTS = """
+import sys
+sys.path.insert(0, %r)
+sys.path.insert(0, %r)
+import slepc_amd as sa
+import test_gpu_sweep as t
+sa.init(0)
+# a single row, one chunk of 128 rows and its neighbours, more chunks than
+# workgroups; basis widths on both sides of every kernel's column limit
+for n, m, prec in ((1, 1, "fp64"), (127, 17, "fp64"), (128, 33, "fp32"), (129, 49, "fp64"), (3001, 66, "fp64"),
+                   (3001, 98, "fp64"), (2999, 126, "fp32"), (65663, 30, "fp64"), (65663, 30, "fp32")):
+    if n == 1:
+        V = sa.BV(1, 2)
+        V.set_column(0, [-3.0])
+        nrm, lindep = V.orthonormalize_column(0)
+        assert nrm == 3.0 and not lindep and V.get_column(0)[0] == -1.0
+        continue
+    t.check_relation(sa, n, min(m, n - 1), "band", prec)
+    print(n, m, prec, flush=True)
+"""
+
+
+def test_slots_relation():
+    """The same relation slot by slot (csrc/sa_gw.hip)."""
+    env = dict(os.environ, SLEPC_AMD_SWEEP_POLLS="0")
+    subprocess.run([sys.executable, "-c", SLOTS % (ROOT, os.path.join(ROOT, "tests"))], check=True, env=env,
+                   timeout=100)
+
+
+def test_slots_relation_large(sa):
+    """Beyond the registers' capacity, no override needed."""
+    check_relation(sa, 200001, 64, "band", "fp64")
 
 
 def test_sweep_gives_up_and_starts_over(tmp_path):

@@ -108,15 +108,14 @@ __device__ __forceinline__ T scatter_add(T x, T y, int lane) {
   }
 }
 // Reduce-scatter of p[0..N) over the wave (N a power of two up to 64): lane l
-// returns the sum over the lanes of p[l / (64 / N)].
-template <int N, int M = 32, typename T>
-__device__ __forceinline__ T wave_scatter(T (&p)[N], int lane) {
-  constexpr int H = N * M / 64;            // values each lane keeps after this step
-  if constexpr (H >= 1) {
+// returns the sum over the lanes of p[l / (64 / N)].  With M below 32 the steps
+// above it have been taken: N values are left for the 2M lanes of a group.
+template <int N, int M = 32, int CAP, typename T>
+__device__ __forceinline__ T wave_scatter(T (&p)[CAP], int lane) {
+  if constexpr (N > 1) {
 #pragma unroll
-    for (int i = 0; i < H; i++) p[i] = scatter_add<M>(p[i], p[i + H], lane);
-    if constexpr (M > 1) return wave_scatter<N, M / 2>(p, lane);
-    else return p[0];
+    for (int i = 0; i < N / 2; i++) p[i] = scatter_add<M>(p[i], p[i + N / 2], lane);
+    return wave_scatter<N / 2, M / 2>(p, lane);
   } else {
     return lanes_sum<2 * M>(p[0]);
   }

@@ -315,3 +315,29 @@ def test_bv_matmult_stream_layout_oracle(sa, orc):
     Y = sa.BV(n, 9, 0)
     X.matmult(A, Y)
     assert np.array_equal(Y.get_matrix(9), orc.bv_matmult(Ao, Xh))
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,k", [(1, 1), (8, 8), (40, 33), (64, 64), (511, 25), (512, 32), (513, 32), (1023, 16),
+                                 (1025, 9), (513, 49), (545, 33), (1057, 24), (16385, 17), (33000, 48)])
+def test_tsqr_tile_edges(sa, n, k, prec):
+    """Tiles of 512 and 1024 rows and their neighbours, a last tile with one
+    row or fewer rows than columns, block widths on both sides of every
+    kernel's column limit: R and Q equal numpy's (geqrf/orgqr, signs included).
+    Perturbations of relative size p (about 10 rounding errors per column)
+    change R and Q by at most p times the condition number."""
+    P = sa.FP64 if prec == "fp64" else sa.FP32
+    eps = EPS if prec == "fp64" else 6e-8
+    rng = np.random.default_rng(17 * n + k)
+    X = rng.standard_normal((n, k))
+    if prec == "fp32":
+        X = X.astype(np.float32).astype(np.float64)
+    V = sa.BV(n, k, P)
+    V.set_matrix(X)
+    R = V.orthogonalize("tsqr")
+    Q = V.get_matrix(k)
+    Qr, Rr = np.linalg.qr(X)
+    tol = 10 * k * eps * np.linalg.cond(X)
+    assert np.linalg.norm(R - Rr) <= tol * np.linalg.norm(Rr)
+    assert np.linalg.norm(Q - Qr) <= tol * np.sqrt(k)
+    assert np.linalg.norm(Q.T @ Q - np.eye(k)) <= 20 * k * eps

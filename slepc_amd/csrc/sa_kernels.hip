@@ -367,31 +367,40 @@ __global__ __launch_bounds__(BLK) void multinplace_kernel(int64_t n, int64_t ld,
 }
 
 // Restart GEMM with Q staged in LDS (used when Q(l:k,s:e) fits in MIP_QS_BYTES).
-// The workgroup converts Q(l:k, s:e) to T in LDS once, then strides over
-// 64-row blocks; wave w computes rows 16w..16w+15 of a block for all N
-// columns.  The MFMA computes the transposed tile, C^T(j, i) = sum_k Q(k, j)
-// V(i, k): operand A is Q from LDS, operand B the basis values, loaded
-// straight from HBM (lanes 0-15 read 16 consecutive rows of one column) in
-// batches of MIP_KB k-steps with the next batch in flight.  Output element v
-// of a lane is column j = 4g+v (f32) or g+4v (f64) of the tile, g = lane/16,
-// and row i = lane%16, so a store writes 128-byte runs of a column.  Every
-// wave reads all K basis values of its rows before it writes them, and no
-// other wave touches those rows, so the product is safe in place.  A basis
+// The workgroup converts Q(l:k, s:e) to T in LDS once; its waves then stride
+// over blocks of 16 VL rows (VL rows of 16 bytes per lane: 2 in FP64, 4 in FP32)
+// and compute all N columns of theirs.  The MFMA computes transposed tiles, C^T(j,
+// i) = sum_k Q(k, j) V(i, k): operand A is Q from LDS, operand B the basis values,
+// loaded straight from HBM: a lane's 16 bytes are rows VL i .. VL i + VL - 1 of
+// one column, one row for each of VL tiles, so that a load covers 256 bytes of
+// four columns, a Q value from LDS serves VL products and a store writes
+// 16 bytes of a column.  Batches of KB k-steps; the next batch is in flight
+// during the products of the current one, across the blocks too (a block that
+// starts and ends with an empty pipeline loses a third of the rate at K = 96).
+// n = 2.1M: K = 96, N = 48 FP64 596 -> 517 us (2.42 GB at 4.7 TB/s, the rate of a
+// device copy here), FP32 475 -> 297; K = 64, N = 32 FP64 355 -> 335.
+// Every wave reads all K basis values of its rows before it writes them, and
+// no other wave touches those rows, so the product is safe in place.  A basis
 // larger than the last-level cache (NT) is read with non-temporal loads, each
-// value being read once (1.2x faster at K = 32, n = 2.1M; at K = 96 the FP64
-// MFMA work, 2 K N flops per row, is as long as the memory time).
-constexpr int MIP_KB = 8;
+// value being read once.  Output element v of a lane is column j = 4g+v (f32) or
+// g+4v (f64) of the tile, g = lane/16.
 constexpr size_t MIP_QS_BYTES = 64 * 1024;
-constexpr int64_t MIP_GRID = 1024;             // workgroups (each stages Q once)
+// Workgroups (each stages Q once): whole rounds of those that are resident
+// together, four per CU with one row per lane, two of the three that fit with 16
+// bytes, or two rounds of three for short products (1.5M rows, K = 64, N = 32 FP64 with 512, 1024, 1536: 252, 287, 250 us).
+constexpr int64_t MIP_GRID = 1024;
 
-template <typename T, int NTL, bool NT>
+template <typename T, int NTL, int VL, bool NT>
 __global__ __launch_bounds__(BLK) void multinplace_q_kernel(int64_t n, int64_t ld, T *V, int l, int K, int s,
                                                             int N, const double *__restrict__ Q, int ldq) {
   typedef typename Vec4<T>::type V4;
+  constexpr int RW = 16 * VL;                    // rows of a wave's block, VL per lane
+  constexpr int KB = NTL * VL <= 8 ? 8 : 4;      // k-steps per batch
+  typedef T VT __attribute__((ext_vector_type(VL)));
   constexpr int NP = NTL * 16 + 1;               // LDS row stride (odd: rows start in different banks)
   extern __shared__ __align__(16) unsigned char smem_raw[];
   T *Qs = reinterpret_cast<T *>(smem_raw);        // [K4][NP]
-  const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+  const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
   const int K4 = (K + 3) & ~3;
   for (int idx = t; idx < K4 * NTL * 16; idx += BLK) {
     const int kk = idx / (NTL * 16), j = idx % (NTL * 16);
@@ -399,66 +408,104 @@ __global__ __launch_bounds__(BLK) void multinplace_q_kernel(int64_t n, int64_t l
   }
   __syncthreads();
   const int g = lane >> 4, c16 = lane & 15;
-  const int nsteps = K4 / 4, nbatch = (nsteps + MIP_KB - 1) / MIP_KB;
-  const int64_t nblk = (n + CH - 1) / CH;
+  const int nsteps = K4 / 4, nbatch = (nsteps + KB - 1) / KB;
+  const int64_t nblk = (n + RW - 1) / RW, stride = (int64_t)gridDim.x * (BLK / 64);
   constexpr bool kF64 = sizeof(T) == 8;
-  for (int64_t b = blockIdx.x; b < nblk; b += gridDim.x) {
-    const int64_t row = b * CH + w * 16 + c16;
-    const bool rin = row < n;
+  VT av[KB], an[KB];
+  auto fetch = [&](int64_t b, int kb) {
+    const int64_t row = b * RW + c16 * VL;
     const T *src = V + (size_t)l * ld + row;
-    V4 acc[NTL];
+    const bool whole = row + VL <= n;
 #pragma unroll
-    for (int q = 0; q < NTL; q++) acc[q] = (V4){0, 0, 0, 0};
-    T av[MIP_KB], an[MIP_KB];
+    for (int u = 0; u < KB; u++) {
+      const int kk = 4 * (kb * KB + u) + g;
+      an[u] = (VT)(T)0;
+      if (kk < K) {
+        const T *p = src + (size_t)kk * ld;
+        if (whole) {
+          an[u] = ld_stream<NT>(reinterpret_cast<const VT *>(p));
+        } else {
 #pragma unroll
-    for (int u = 0; u < MIP_KB; u++) {
-      const int kk = 4 * u + g;
-      av[u] = (rin && kk < K) ? ld_stream<NT>(src + (size_t)kk * ld) : (T)0;
-    }
-    for (int kb = 0; kb < nbatch; kb++) {
-      if (kb + 1 < nbatch) {
-#pragma unroll
-        for (int u = 0; u < MIP_KB; u++) {
-          const int kk = 4 * ((kb + 1) * MIP_KB + u) + g;
-          an[u] = (rin && kk < K) ? ld_stream<NT>(src + (size_t)kk * ld) : (T)0;
+          for (int e = 0; e < VL; e++)
+            if (row + e < n) an[u][e] = p[e];
         }
       }
+    }
+  };
+  int64_t b = (int64_t)blockIdx.x * (BLK / 64) + w;
+  if (VL > 1 && b < nblk) fetch(b, 0);
+  for (; b < nblk; b += stride) {
+    if (VL == 1) fetch(b, 0);                    // more waves in flight instead
+    V4 acc[VL][NTL];
 #pragma unroll
-      for (int u = 0; u < MIP_KB; u++) {
-        const int step = kb * MIP_KB + u;
+    for (int e = 0; e < VL; e++)
+#pragma unroll
+      for (int q = 0; q < NTL; q++) acc[e][q] = (V4){0, 0, 0, 0};
+    for (int kb = 0; kb < nbatch; kb++) {
+#pragma unroll
+      for (int u = 0; u < KB; u++) av[u] = an[u];
+      if (kb + 1 < nbatch) fetch(b, kb + 1);
+      else if (VL > 1 && b + stride < nblk) fetch(b + stride, 0);
+#pragma unroll
+      for (int u = 0; u < KB; u++) {
+        const int step = kb * KB + u;
         if (step < nsteps) {
           const T *qrow = Qs + (4 * step + g) * NP + c16;
 #pragma unroll
-          for (int q = 0; q < NTL; q++) acc[q] = mfma16x16x4(qrow[q * 16], av[u], acc[q]);
+          for (int q = 0; q < NTL; q++) {
+            const T qv = qrow[q * 16];
+#pragma unroll
+            for (int e = 0; e < VL; e++) acc[e][q] = mfma16x16x4(qv, av[u][e], acc[e][q]);
+          }
         }
       }
-#pragma unroll
-      for (int u = 0; u < MIP_KB; u++) av[u] = an[u];
     }
-    if (rin) {
-      T *dst = V + (size_t)s * ld + row;
+    const int64_t row = b * RW + c16 * VL;
+    T *dst = V + (size_t)s * ld + row;
 #pragma unroll
-      for (int q = 0; q < NTL; q++)
+    for (int q = 0; q < NTL; q++)
 #pragma unroll
-        for (int v = 0; v < 4; v++) {
-          const int j = q * 16 + (kF64 ? (g + 4 * v) : (4 * g + v));
-          if (j < N) dst[(size_t)j * ld] = acc[q][v];
+      for (int v = 0; v < 4; v++) {
+        const int j = q * 16 + (kF64 ? (g + 4 * v) : (4 * g + v));
+        if (j >= N) continue;
+        VT o;
+#pragma unroll
+        for (int e = 0; e < VL; e++) o[e] = acc[e][q][v];
+        if (row + VL <= n) {
+          *reinterpret_cast<VT *>(dst + (size_t)j * ld) = o;
+        } else {
+#pragma unroll
+          for (int e = 0; e < VL; e++)
+            if (row + e < n) dst[(size_t)j * ld + e] = o[e];
         }
-    }
+      }
   }
+}
+
+template <typename T, int NTL, int VL>
+static void launch_mip_rows(BV &V, int l, int K, int s_, int N, const double *Q_dev, int ldq, hipStream_t s) {
+  const int64_t rows = 4 * 16 * VL;                // per workgroup step
+  const int grid = (int)std::min<int64_t>((V.n + rows - 1) / rows, VL == 1 ? MIP_GRID : (NTL == 1 ? 3 * MIP_GRID / 2 : MIP_GRID / 2));
+  const size_t shm = (size_t)((K + 3) & ~3) * (NTL * 16 + 1) * sizeof(T);
+  if (V.n * (int64_t)K * (int64_t)sizeof(T) > GS_NT_BYTES)
+    hipLaunchKernelGGL((multinplace_q_kernel<T, NTL, VL, true>), dim3(grid), dim3(BLK), shm, s, V.n, V.ld,
+                       (T *)V.data, l, K, s_, N, Q_dev, ldq);
+  else
+    hipLaunchKernelGGL((multinplace_q_kernel<T, NTL, VL, false>), dim3(grid), dim3(BLK), shm, s, V.n, V.ld,
+                       (T *)V.data, l, K, s_, N, Q_dev, ldq);
 }
 
 template <typename T, int NTL>
 static void launch_mip_q(BV &V, int l, int K, int s_, int N, const double *Q_dev, int ldq, hipStream_t s) {
-  const int64_t nblk = (V.n + CH - 1) / CH;
-  const int grid = (int)std::min<int64_t>(nblk, MIP_GRID);
-  const size_t shm = (size_t)((K + 3) & ~3) * (NTL * 16 + 1) * sizeof(T);
-  if (V.n * (int64_t)K * (int64_t)sizeof(T) > GS_NT_BYTES)
-    hipLaunchKernelGGL((multinplace_q_kernel<T, NTL, true>), dim3(grid), dim3(BLK), shm, s, V.n, V.ld, (T *)V.data,
-                       l, K, s_, N, Q_dev, ldq);
-  else
-    hipLaunchKernelGGL((multinplace_q_kernel<T, NTL, false>), dim3(grid), dim3(BLK), shm, s, V.n, V.ld, (T *)V.data,
-                       l, K, s_, N, Q_dev, ldq);
+  constexpr int VL = 16 / (int)sizeof(T);
+  // 16 bytes per lane, or one row per lane for few output columns and on small
+  // blocks, where more waves count (microseconds with 16 bytes and with one row, FP64:
+  // K = 30, N = 15 at 1.5M rows 106.8, 108.3, K = 20, N = 10 at 300,000 32.8, 30.4; K = 32,
+  // N = 16 at 30,000 23.6, 22.1; K = 90, N = 48 at 50,000 50.9, 52.1, at 100,000 61.6,
+  // 66.6; FP32 four rows per lane: at 100,000 53.2, 50.4)
+  constexpr int shift = sizeof(T) == 8 ? (NTL > 1 ? 22 : 25) : (NTL > 1 ? 24 : 62);
+  if (V.n * K >= (int64_t)1 << shift) launch_mip_rows<T, NTL, VL>(V, l, K, s_, N, Q_dev, ldq, s);
+  else launch_mip_rows<T, NTL, 1>(V, l, K, s_, N, Q_dev, ldq, s);
 }
 
 template <typename T>

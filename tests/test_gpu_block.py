@@ -341,3 +341,25 @@ def test_tsqr_tile_edges(sa, n, k, prec):
     assert np.linalg.norm(R - Rr) <= tol * np.linalg.norm(Rr)
     assert np.linalg.norm(Q - Qr) <= tol * np.sqrt(k)
     assert np.linalg.norm(Q.T @ Q - np.eye(k)) <= 20 * k * eps
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,K,N", [(15, 5, 3), (65, 33, 17), (65537, 33, 16), (66049, 40, 49), (131201, 20, 7),
+                                   (140003, 96, 48)])
+def test_restart_product_row_blocks(sa, n, K, N, prec):
+    """BVMultInPlace at the edges of its row blocks (one row per lane, 16 bytes
+    per lane from 65,536 rows on, ragged last blocks, more blocks than
+    workgroups) against the product in FP64: K rounded products per entry."""
+    P = sa.FP64 if prec == "fp64" else sa.FP32
+    eps = EPS if prec == "fp64" else 6e-8
+    rng = np.random.default_rng(n + K)
+    X = rng.uniform(-1.0, 1.0, (n, K)).astype(np.float32).astype(np.float64)
+    Q = rng.uniform(-1.0, 1.0, (K, K)).astype(np.float32).astype(np.float64)
+    N = min(N, K)
+    V = sa.BV(n, K, P)
+    V.set_matrix(X)
+    V.set_active_columns(0, K)
+    V.multinplace(Q, 0, N)
+    Y = V.get_matrix(K)
+    assert np.abs(Y[:, :N] - X @ Q[:, :N]).max() <= K * K * eps
+    assert np.array_equal(Y[:, N:], X[:, N:])

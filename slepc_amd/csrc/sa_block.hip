@@ -10,7 +10,10 @@ namespace sa {
 
 // ---------------------------------------------------------------------------
 // BVDot: M(i, j) = Y(:, i) . X(:, j), i < my <= 64, j < mx <= 64.  A
-// workgroup walks its rows in 32-row chunks, stages the chunk of both
+// workgroup walks 32-row chunks in grid-stride order (the workgroups in flight
+// then read one contiguous stretch of every column; a contiguous range of rows
+// per workgroup measured 241 us where this takes 207, two 32-column blocks of
+// 2.1M rows: 5.2 TB/s), stages the chunk of both
 // blocks in LDS (stride 33: the 16 lanes of a tile row read 16 columns of
 // one row without bank conflicts) and accumulates 16x16 tiles of M with
 // MFMA 16x16x4 (operand A = Y^T, operand B = X); wave w owns tiles w, w+4,
@@ -19,19 +22,20 @@ namespace sa {
 // ---------------------------------------------------------------------------
 constexpr int BD_ROWS = 32, BD_LDP = BD_ROWS + 1, BD_MAXC = 64, BD_MAXG = 1024;
 
-template <typename T, bool NT, int PC>
-__global__ __launch_bounds__(BLK) void bvdot_kernel(int64_t n, int64_t rpb, const T *__restrict__ X, int64_t ldx,
+template <typename T, bool NT, int PC, bool SAME>
+__global__ __launch_bounds__(BLK) void bvdot_kernel(int64_t n, const T *__restrict__ X, int64_t ldx,
                                                     int mx, const T *__restrict__ Y, int64_t ldy, int my,
                                                     double *__restrict__ part, int G) {
   typedef typename Vec4<T>::type V4;
   __shared__ T Ys[PC * (BLK / BD_ROWS) * BD_LDP];   // tiles sized for the columns handled
-  __shared__ T Xs[PC * (BLK / BD_ROWS) * BD_LDP];
+  __shared__ T Xt[SAME ? 1 : PC * (BLK / BD_ROWS) * BD_LDP];
+  T *Xs = SAME ? Ys : Xt;                           // Gram matrix of one block: staged once
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, g = lane >> 4, c16 = lane & 15;
   const int nty = (my + 15) / 16, ntx = (mx + 15) / 16, ntile = nty * ntx;
   V4 acc[4];
 #pragma unroll
   for (int q = 0; q < 4; q++) acc[q] = (V4){0, 0, 0, 0};
-  const int64_t rb = (int64_t)blockIdx.x * rpb, re = min(n, rb + rpb);
+  const int64_t rb = (int64_t)blockIdx.x * BD_ROWS, stp = (int64_t)G * BD_ROWS;
   const int row = t & (BD_ROWS - 1), cg = t / BD_ROWS;      // 8 column groups
   static_assert(PC * (BLK / BD_ROWS) <= BD_MAXC, "columns per thread and block");
   // register double buffer: the next chunk's loads are in flight while the
@@ -39,24 +43,24 @@ __global__ __launch_bounds__(BLK) void bvdot_kernel(int64_t n, int64_t rpb, cons
   // extra registers halve the occupancy)
   T py[PC], px[PC];
   auto fetch = [&](int64_t r0) {
-    const bool in = r0 + row < re;
+    const bool in = r0 + row < n;
 #pragma unroll
     for (int q = 0; q < PC; q++) {
       const int i = cg + q * (BLK / BD_ROWS);
       py[q] = (in && i < my) ? tile_load<NT>(Y + (size_t)i * ldy + r0 + row) : (T)0;
-      px[q] = (in && i < mx) ? tile_load<NT>(X + (size_t)i * ldx + r0 + row) : (T)0;
+      if constexpr (!SAME) px[q] = (in && i < mx) ? tile_load<NT>(X + (size_t)i * ldx + r0 + row) : (T)0;
     }
   };
-  if (rb < re) fetch(rb);
-  for (int64_t r0 = rb; r0 < re; r0 += BD_ROWS) {
+  if (rb < n) fetch(rb);
+  for (int64_t r0 = rb; r0 < n; r0 += stp) {
 #pragma unroll
     for (int q = 0; q < PC; q++) {
       const int i = cg + q * (BLK / BD_ROWS);
       if (i < my) Ys[i * BD_LDP + row] = py[q];
-      if (i < mx) Xs[i * BD_LDP + row] = px[q];
+      if (!SAME && i < mx) Xs[i * BD_LDP + row] = px[q];
     }
     __syncthreads();
-    if (r0 + BD_ROWS < re) fetch(r0 + BD_ROWS);
+    if (r0 + stp < n) fetch(r0 + stp);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
       const int tile = w + 4 * q;
@@ -93,7 +97,7 @@ __global__ __launch_bounds__(BLK) void bvdot_sum_kernel(const double *part, int 
 }
 
 template <typename T>
-static int bvdot_block(const BV &X, int lx, int mx, const BV &Y, int ly, int my, double *part, int G, int64_t rpb,
+static int bvdot_block(const BV &X, int lx, int mx, const BV &Y, int ly, int my, double *part, int G,
                        double *out, hipStream_t s) {
   const T *xp = static_cast<const T *>(X.data) + (size_t)lx * X.ld;
   const T *yp = static_cast<const T *>(Y.data) + (size_t)ly * Y.ld;
@@ -102,14 +106,25 @@ static int bvdot_block(const BV &X, int lx, int mx, const BV &Y, int ly, int my,
   // registers for 4 columns per thread and block when both blocks have at
   // most 32 columns (the occupancy the loads in flight need), else 8
   const bool narrow = mx <= 4 * (BLK / BD_ROWS) && my <= 4 * (BLK / BD_ROWS);
-  if (nt && narrow)
-    hipLaunchKernelGGL((bvdot_kernel<T, true, 4>), dim3(G), dim3(BLK), 0, s, X.n, rpb, xp, X.ld, mx, yp, Y.ld, my, part, G);
-  else if (nt)
-    hipLaunchKernelGGL((bvdot_kernel<T, true, 8>), dim3(G), dim3(BLK), 0, s, X.n, rpb, xp, X.ld, mx, yp, Y.ld, my, part, G);
-  else if (narrow)
-    hipLaunchKernelGGL((bvdot_kernel<T, false, 4>), dim3(G), dim3(BLK), 0, s, X.n, rpb, xp, X.ld, mx, yp, Y.ld, my, part, G);
-  else
-    hipLaunchKernelGGL((bvdot_kernel<T, false, 8>), dim3(G), dim3(BLK), 0, s, X.n, rpb, xp, X.ld, mx, yp, Y.ld, my, part, G);
+  const bool same = xp == yp && mx == my;
+  // Workgroups (2.1M rows, microseconds with 512, 768, 1024): FP64 64 columns 575, 528,
+  // 599; 32 columns 212, 220, 226; 24 columns 201, 172, 172; FP32 64 columns 423, 378, 373; one
+  // block with itself, FP64 64 columns 488, 442, 424, 32 columns 183, 161, 150 (staged
+  // twice: 217).
+  const int most = same || sizeof(T) == 4 ? BD_MAXG : (mx > 32 || my > 32 ? 768 : (mx + my > 48 ? 512 : BD_MAXG));
+  G = std::min(G, most);
+  auto go = [&](auto *kern) { hipLaunchKernelGGL(kern, dim3(G), dim3(BLK), 0, s, X.n, xp, X.ld, mx, yp, Y.ld, my, part, G); };
+  if (same) {
+    if (nt && narrow) go(bvdot_kernel<T, true, 4, true>);
+    else if (nt) go(bvdot_kernel<T, true, 8, true>);
+    else if (narrow) go(bvdot_kernel<T, false, 4, true>);
+    else go(bvdot_kernel<T, false, 8, true>);
+  } else {
+    if (nt && narrow) go(bvdot_kernel<T, true, 4, false>);
+    else if (nt) go(bvdot_kernel<T, true, 8, false>);
+    else if (narrow) go(bvdot_kernel<T, false, 4, false>);
+    else go(bvdot_kernel<T, false, 8, false>);
+  }
   hipLaunchKernelGGL(bvdot_sum_kernel, dim3(my * mx), dim3(BLK), 0, s, (const double *)part, G, out);
   SA_HIP(hipGetLastError());
   return 0;
@@ -130,7 +145,6 @@ int launch_bvdot(const BV &X, int lx, int kx, const BV &Y, int ly, int ky, doubl
   SA_CHECK(X.prec == Y.prec && X.n == Y.n, "BVDot: bases differ in length or precision");
   const int64_t chunks = std::max<int64_t>(1, (X.n + BD_ROWS - 1) / BD_ROWS);
   const int G = (int)std::min<int64_t>(BD_MAXG, chunks);
-  const int64_t rpb = (chunks + G - 1) / G * BD_ROWS;
   thread_local BdWork W;
   if (W.G < G) {
     if (W.part) (void)hipFree(W.part);
@@ -146,8 +160,8 @@ int launch_bvdot(const BV &X, int lx, int kx, const BV &Y, int ly, int ky, doubl
   for (int bj = 0; bj < mx && !rc; bj += BD_MAXC)
     for (int bi = 0; bi < my && !rc; bi += BD_MAXC) {
       const int nx = std::min(BD_MAXC, mx - bj), ny = std::min(BD_MAXC, my - bi);
-      rc = X.prec == SA_FP64 ? bvdot_block<double>(X, lx + bj, nx, Y, ly + bi, ny, part, G, rpb, blk, s)
-                             : bvdot_block<float>(X, lx + bj, nx, Y, ly + bi, ny, part, G, rpb, blk, s);
+      rc = X.prec == SA_FP64 ? bvdot_block<double>(X, lx + bj, nx, Y, ly + bi, ny, part, G, blk, s)
+                             : bvdot_block<float>(X, lx + bj, nx, Y, ly + bi, ny, part, G, blk, s);
       if (!rc && hipMemcpy2DAsync(M_dev + bi + (size_t)bj * my, sizeof(double) * my, blk, sizeof(double) * ny,
                                   sizeof(double) * ny, nx, hipMemcpyDeviceToDevice, s) != hipSuccess)
         rc = 1;
@@ -158,41 +172,41 @@ int launch_bvdot(const BV &X, int lx, int kx, const BV &Y, int ly, int ky, doubl
 }
 
 // ---------------------------------------------------------------------------
-// BVMatMult: Y(:, j) = A X(:, j) for j < nc <= SPMM_NC.  L lanes per row;
+// BVMatMult: Y(:, j) = A X(:, j) for j < nc <= NC.  L lanes per row;
 // each nonzero's value and column index are loaded once and applied to the
-// nc columns, so the operator is read once per SPMM_NC columns.  The sum of
+// nc columns, so the operator is read once per pass.  The sum of
 // each column runs in the order of the vector-CSR SpMV.  Operators larger
 // than the caches take the stream layout below instead.
 // ---------------------------------------------------------------------------
-constexpr int SPMM_NC = 8;
+constexpr int SPMM_NC = 16;   // columns per pass: 16, 8 or 4
 
-template <typename T, int L>
+template <typename T, int L, int NC>
 __global__ __launch_bounds__(BLK) void spmm_kernel(int n, const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
                                                    const T *__restrict__ val, const T *__restrict__ X, int64_t ldx,
                                                    T *__restrict__ Y, int64_t ldy, int nc) {
   const int lg = threadIdx.x % L;
   const int64_t row = ((int64_t)blockIdx.x * BLK + threadIdx.x) / L;
-  T s[SPMM_NC];
+  T s[NC];
 #pragma unroll
-  for (int j = 0; j < SPMM_NC; j++) s[j] = (T)0;
+  for (int j = 0; j < NC; j++) s[j] = (T)0;
   if (row < n) {
     const int32_t pe = rp[row + 1];
     for (int32_t p = rp[row] + lg; p < pe; p += L) {
       const T v = val[p];
       const int32_t c = ci[p];
 #pragma unroll
-      for (int j = 0; j < SPMM_NC; j++)
+      for (int j = 0; j < NC; j++)
         if (j < nc) s[j] += v * X[(size_t)j * ldx + c];
     }
   }
   // every lane of the group ends with each column's sum; lane q keeps the
-  // columns q, q+L, ... so the stores need SPMM_NC/L instructions, not SPMM_NC
-  constexpr int NS = (SPMM_NC + L - 1) / L;
+  // columns q, q+L, ... so the stores need NC/L instructions, not NC
+  constexpr int NS = (NC + L - 1) / L;
   T mine[NS];
 #pragma unroll
   for (int u = 0; u < NS; u++) mine[u] = (T)0;
 #pragma unroll
-  for (int j = 0; j < SPMM_NC; j++) {
+  for (int j = 0; j < NC; j++) {
     T sj = s[j];
 #pragma unroll
     for (int off = L / 2; off > 0; off >>= 1) sj += __shfl_xor(sj, off, L);
@@ -221,7 +235,7 @@ __global__ __launch_bounds__(BLK) void spmm_kernel(int n, const int32_t *__restr
 // columns, into TPR strided partial sums per column (nonzero p goes to sum
 // (p - b) % TPR, in order).  The nonzeros are taken TPR at a time: their
 // values and indices first (indices clamped to the row, so every load is in
-// bounds), then all their gathers of x (TPR * NCT = SPMM_NC loads in flight),
+// bounds), then all their gathers of x (TPR * NCT = NC loads in flight),
 // then the sums.  Batches of 2 or 4 times as many nonzeros measured slower at
 // 128^3 on the 27-point operator (more x in flight than the L2 holds).
 // Products are rounded before they are added, as in the stream SpMV.
@@ -257,14 +271,14 @@ __device__ __forceinline__ void spmm_row(VP vs, CP cs, int b, int e, const T *co
   }
 }
 
-template <typename T, int RB>
+template <typename T, int RB, int NC>
 __global__ __launch_bounds__(BLK) void spmm_stream_kernel(int n, const int32_t *__restrict__ rp,
                                                           const int32_t *__restrict__ ci, const T *__restrict__ val,
                                                           const T *__restrict__ X, int64_t ldx, T *__restrict__ Y,
                                                           int64_t ldy, int nc) {
   constexpr int TPR = BLK / RB;
-  constexpr int NCT = SPMM_NC / TPR;   // columns per thread
-  static_assert(RB <= BLK && BLK % RB == 0 && SPMM_NC % TPR == 0, "row block");
+  constexpr int NCT = NC / TPR;   // columns per thread
+  static_assert(RB <= BLK && BLK % RB == 0 && NC % TPR == 0, "row block");
   __shared__ T sval[SPMV_NZB];
   __shared__ int32_t scol[SPMV_NZB];
   __shared__ int32_t srp[RB + 1];
@@ -302,27 +316,39 @@ __global__ __launch_bounds__(BLK) void spmm_stream_kernel(int n, const int32_t *
   }
 }
 
-template <typename T>
+template <typename T, int NC>
 static void spmm_t(const Mat &A, const T *X, int64_t ldx, T *Y, int64_t ldy, int nc, hipStream_t s) {
+  const T *val = static_cast<const T *>(A.val);
   if (A.spmv_rb > 0) {   // operators larger than the caches: the stream layout
     const int grid = (int)(((int64_t)A.n + A.spmv_rb - 1) / A.spmv_rb);
-    const T *val = static_cast<const T *>(A.val);
+    auto go = [&](auto *kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); };
     switch (A.spmv_rb) {
-      case 256: hipLaunchKernelGGL((spmm_stream_kernel<T, 256>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
-      case 128: hipLaunchKernelGGL((spmm_stream_kernel<T, 128>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
-      case 64: hipLaunchKernelGGL((spmm_stream_kernel<T, 64>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
-      default: hipLaunchKernelGGL((spmm_stream_kernel<T, 32>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
+      case 256: go(spmm_stream_kernel<T, 256, NC>); break;
+      case 128: go(spmm_stream_kernel<T, 128, NC>); break;
+      case 64: go(spmm_stream_kernel<T, 64, NC>); break;
+      default: go(spmm_stream_kernel<T, 32, (NC < 8 ? 8 : NC)>); break;
     }
     return;
   }
   const int grid = (int)(((int64_t)A.n * A.lanes + BLK - 1) / BLK);
-  const T *val = static_cast<const T *>(A.val);
+  auto go = [&](auto *kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); };
   switch (A.lanes) {
-    case 4: hipLaunchKernelGGL((spmm_kernel<T, 4>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
-    case 8: hipLaunchKernelGGL((spmm_kernel<T, 8>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
-    case 16: hipLaunchKernelGGL((spmm_kernel<T, 16>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
-    default: hipLaunchKernelGGL((spmm_kernel<T, 32>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, X, ldx, Y, ldy, nc); break;
+    case 4: go(spmm_kernel<T, 4, NC>); break;
+    case 8: go(spmm_kernel<T, 8, NC>); break;
+    case 16: go(spmm_kernel<T, 16, NC>); break;
+    default: go(spmm_kernel<T, 32, NC>); break;
   }
+}
+
+// A pass takes 16 columns, the last one the fewest of 16, 8 and 4 that hold the
+// rest (a column beyond the rest costs its gathers).  32 columns at 128^3 with
+// passes of 8, 16, 32: 7-point 530, 490, 475 us, 27-point 1426, 1304, 1323;
+// 900,000 rows 5-point 399, 386, 669.
+template <typename T>
+static void spmm_cols(const Mat &A, const T *X, int64_t ldx, T *Y, int64_t ldy, int nc, hipStream_t s) {
+  if (nc > 8) spmm_t<T, 16>(A, X, ldx, Y, ldy, nc, s);
+  else if (nc > 4) spmm_t<T, 8>(A, X, ldx, Y, ldy, nc, s);
+  else spmm_t<T, 4>(A, X, ldx, Y, ldy, nc, s);
 }
 
 int launch_spmm(const Mat &A, const BV &X, int lx, const BV &Y, int ly, int ncols, hipStream_t s) {
@@ -334,11 +360,11 @@ int launch_spmm(const Mat &A, const BV &X, int lx, const BV &Y, int ly, int ncol
     if (X.prec == SA_FP64) {
       const double *xp = static_cast<const double *>(X.data) + (size_t)(lx + j0) * X.ld;
       double *yp = static_cast<double *>(Y.data) + (size_t)(ly + j0) * Y.ld;
-      spmm_t<double>(A, xp, X.ld, yp, Y.ld, nc, s);
+      spmm_cols<double>(A, xp, X.ld, yp, Y.ld, nc, s);
     } else {
       const float *xp = static_cast<const float *>(X.data) + (size_t)(lx + j0) * X.ld;
       float *yp = static_cast<float *>(Y.data) + (size_t)(ly + j0) * Y.ld;
-      spmm_t<float>(A, xp, X.ld, yp, Y.ld, nc, s);
+      spmm_cols<float>(A, xp, X.ld, yp, Y.ld, nc, s);
     }
   }
   SA_HIP(hipGetLastError());

@@ -363,3 +363,26 @@ def test_restart_product_row_blocks(sa, n, K, N, prec):
     Y = V.get_matrix(K)
     assert np.abs(Y[:, :N] - X @ Q[:, :N]).max() <= K * K * eps
     assert np.array_equal(Y[:, N:], X[:, N:])
+
+
+@pytest.mark.parametrize("nc", [1, 4, 5, 8, 9, 16, 17, 20, 40])
+def test_matmult_column_passes(sa, nc):
+    """BVMatMult in passes of 16, 8 and 4 columns, on a small operator and in the
+    stream layout: every column equals MatMult bit for bit there, and to rounding
+    on the small one; BVDot over more chunks than workgroups."""
+    A = sa.stencil27(23, 19, 17)
+    rng = np.random.default_rng(nc)
+    X = rng.uniform(-1.0, 1.0, (A.n, nc))
+    for thr in (None, 0):
+        prev = sa.set_spmv_stream_bytes(0) if thr == 0 else None
+        M = sa.Mat(A)
+        if prev is not None:
+            sa.set_spmv_stream_bytes(prev)
+        V, W = sa.BV(A.n, nc), sa.BV(A.n, nc)
+        V.set_matrix(X)
+        V.matmult(M, W)
+        Y = W.get_matrix(nc)
+        Z = np.stack([M.mult_host(X[:, j]) for j in range(nc)], axis=1)
+        assert np.array_equal(Y, Z) if thr == 0 else np.abs(Y - Z).max() <= 64 * EPS * np.abs(Z).max()
+        G = V.dot(W)
+        assert np.abs(G - Y.T @ X).max() <= 200 * EPS * np.linalg.norm(X, axis=0).max() * np.linalg.norm(Y, axis=0).max()

@@ -573,9 +573,11 @@ int ps_go(BV &V, const Mat *A, PsArgs<T> &a, hipStream_t s) {
     // the rows' nonzeros with a quarter to spare (at least one more than the
     // room allows is caught in the kernel), up to 4 remote entries per row, and
     // in the same memory at set-up two bits per column of their span
-    a.hcap = std::min(4 * R, 4096);
-    const size_t rest = room - (size_t)a.hcap * (sizeof(T) + 4);
+    // room / 4 at least goes to the remote entries, what the rows leave to them
     const size_t nz = (size_t)(1.25 * (double)A->nnz / (double)std::max(1, A->n) * R) + 64;
+    const size_t left = room - std::min(nz * (sizeof(T) + 2), room - room / 4);
+    a.hcap = (int)std::min({(size_t)4 * R, (size_t)4096, left / (sizeof(T) + 4)}) & ~1;
+    const size_t rest = room - (size_t)a.hcap * (sizeof(T) + 4);
     a.nzcap = (int)(std::min(nz, rest / (sizeof(T) + 2)) & ~(size_t)1);
     shm = (size_t)a.nzcap * (sizeof(T) + 2) + (size_t)a.hcap * (sizeof(T) + 4);
     const size_t span = ((size_t)V.n + 31) / 32 * 32;
@@ -618,15 +620,12 @@ template <typename T>
 int ps_pick(int64_t n, int S, int share) {
   constexpr int M = sizeof(T) == 8 ? 88 : 176;
   const int most = std::min(num_cus(), 64 * PS_D);
-  const int want = share >= 2 ? std::max(64, most / 2) : most;
-  int best = 0;
-  for (int q : {1, 2, 4, 6, 8, 11, 16, 22}) {
-    const int64_t G = (n + 64 * q - 1) / (64 * q);
-    if (S * q > M || G > most) continue;
-    best = q;
-    if (G <= want && (G <= 64 || q >= 4)) break;
-  }
-  return best;
+  for (int want : {share >= 2 ? std::max(64, most / 2) : most, most})
+    for (int q : {1, 2, 4, 6, 8, 11, 16, 22}) {
+      const int64_t G = (n + 64 * q - 1) / (64 * q);
+      if (S * q <= M && G <= want && (G <= 64 || q >= 4)) return q;
+    }
+  return 0;
 }
 
 // Polls before a wait gives up: about half a second, or SLEPC_AMD_SWEEP_POLLS

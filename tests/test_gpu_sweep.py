@@ -75,6 +75,19 @@ def test_sweep_relation(sa, n, m, kind, prec):
     check_relation(sa, n, m, kind, prec)
 
 
+@pytest.mark.parametrize("n,m,kind,prec", [
+    (180225, 12, "band", "fp64"), (200001, 32, "band", "fp64"), (131073, 33, "ragged", "fp64"),
+    (65537, 40, "band", "fp64"), (260000, 30, "band", "fp32")])
+def test_sweep_relation_half_the_workgroups(sa, n, m, kind, prec):
+    """With other solves announced the sweep takes half the CUs where they hold
+    the basis, and all of them where they do not."""
+    before = sa.set_concurrent_solves(2)
+    try:
+        check_relation(sa, n, m, kind, prec)
+    finally:
+        sa.set_concurrent_solves(max(1, before))
+
+
 CODE = """
 import sys, numpy as np
 sys.path.insert(0, %r)

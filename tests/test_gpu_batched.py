@@ -45,6 +45,25 @@ def test_batched_matches_oracle(sa, orc, mixed, sweep):
     assert st["matvecs"] > 0 and (st["matvecs32"] > 0) == mixed
 
 
+@pytest.mark.parametrize("P", [1, 7, 8, 9, 33])
+def test_batched_projected_problems_on_host_threads(sa, orc, P):
+    """From 8 problems on the projected problems go to the solve's own host
+    threads; problems that converge early leave fewer than 8 to the later
+    rounds.  Every problem's values are the oracle's."""
+    from slepc_amd.batch import Batch, uneven_laplacians
+    csrs = uneven_laplacians(P=P, seed=5, lo=12, hi=40)
+    v0 = [orc.rand_uniform(orc.sub_seed(3, p), A.n) for p, A in enumerate(csrs)]
+    B = Batch(csrs)
+    for _ in range(2):
+        B.solve(4, 16, 1e-10, "LM", v0=v0)
+        for p, A in enumerate(csrs):
+            assert B.converged(p)[2] == 1
+            w = np.linalg.eigvalsh(orc.CSR(A.n, A.rowptr, A.col, A.val).to_dense())
+            for i in range(4):
+                v = B.eigenpair(p, i, False)[0]
+                assert np.min(np.abs(w - v)) < 1e-10 * abs(v)
+
+
 def test_batched_c5_shapes(sa):
     """The 512-problem family: sizes span 1k..65k rows and all converge."""
     from slepc_amd.batch import Batch, uneven_laplacians

@@ -1,6 +1,6 @@
 """Batched Krylov-Schur over many independent symmetric problems (C ABI
 sa_batch_*): one block-diagonal operator, one basis; each restart sweep is
-either one launch with a workgroup per problem, or lock-step launches per
+either one launch with workgroups of its own per problem, or lock-step launches per
 Gram-Schmidt slot over the row chunks of all problems (autotuned)."""
 import ctypes as C
 
@@ -103,7 +103,7 @@ class Batch:
 
     def set_sweep(self, mode):
         """"auto" (time both sweep kernels on the first restart round), "persistent"
-        (a workgroup per problem, ncv < 64) or "wide" (lock-step over row chunks)."""
+        (resident: workgroups of its own per problem, ncv < 64) or "wide" (lock-step over row chunks)."""
         check(self.L.sa_batch_set_sweep(self.h, SWEEP_MODES[mode]))
 
     def sweep_info(self):
@@ -114,7 +114,7 @@ class Batch:
 
     def schedule(self):
         """The last solve's sweep schedule and the autotuner's timings (ms) of the
-        candidates [one workgroup per problem, lock-step, other tile loads,
+        candidates [resident, lock-step, other tile loads,
         twice the SpMV lanes] (-1: not timed)."""
         k, nt, la = C.c_int(), C.c_int(), C.c_int()
         ms = np.zeros(4)

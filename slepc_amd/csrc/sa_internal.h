@@ -87,6 +87,22 @@ struct PsWork {              // exchange words of the resident sweep (sa_sweep.h
   int share = 1;             // sa_set_concurrent_solves when the basis was created
 };
 
+struct PsProb {              // one problem of a batched resident sweep
+  int64_t n0, n1;            // its rows of the stacked basis
+  int c0, c1;                // columns to compute
+  int id;                    // its place in the states and coefficients
+  int G, b0;                 // its workgroups (set by the launch)
+};
+
+struct PsBatch {             // device state of the batched resident sweep
+  uint64_t *words = nullptr;             // exchange words: vector, partial sums, totals, abort word
+  size_t pw = 0, tw = 0, abort_word = 0, bytes = 0;
+  uint32_t tag = 1;
+  PsProb *probs = nullptr;
+  int *of_block = nullptr;
+  GsMirror *fail = nullptr;              // pinned
+};
+
 struct BV {
   int64_t n = 0, ld = 0;
   int m = 0, prec = SA_FP64;
@@ -138,6 +154,15 @@ int launch_gs_reset(BV &V, hipStream_t s);
 // Blocks on the stream.
 int ps_sweep(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool *done);
 size_t ps_bytes(int64_t n, int prec);   // bytes of its exchange words, 0 when no basis of n rows fits
+// The sweeps of several problems (rows stacked in one basis, block-diagonal
+// operator) in as few launches as the CUs allow; *done is false when one does
+// not fit or gave up (columns c0 .. c1 and the states are then undefined).
+// Blocks on the stream.
+bool ps_batch_alloc(PsBatch &w, int64_t nrows, int prec, int P, hipStream_t s);   // false: no memory
+void ps_batch_free(PsBatch &w);
+int ps_batch_sweep(PsBatch &w, int prec, void *V, int64_t ld, int64_t nrows, const int32_t *rp, const int32_t *ci,
+                   const void *val, int64_t nnz, std::vector<PsProb> &pr, GsState *st, double *dbuf, int m, double eta,
+                   hipStream_t s, bool *done);
 int concurrent_solves();      // the application's hint (sa_set_concurrent_solves)
 int gw_blocks(int64_t n, int prec, int c);   // workgroups of a Gram-Schmidt slot of column c (sa_gw.hip)
 int launch_dotvec(BV &V, int l, int k, const void *x, double *q_dev, hipStream_t s);

@@ -51,6 +51,7 @@
 #include <condition_variable>
 #include <cstdlib>
 #include <mutex>
+#include <vector>
 
 #include "sa_gs_device.h"
 
@@ -66,7 +67,8 @@ constexpr int PS_COPIES = 8;            // copies of the totals
 
 template <typename T>
 struct PsArgs {
-  int64_t n, ld;
+  int64_t n0, n1;             // the rows it computes: n0 .. n1 - 1 (operator columns and words count from 0)
+  int64_t xn, ld;             // words of a vector's low halves, stride of the basis
   T *V;
   const int32_t *rp, *ci;     // operator, or null: column c0 itself is orthonormalised
   const T *val;
@@ -122,7 +124,7 @@ __device__ __forceinline__ bool ps_gather(const PsArgs<T> &a, const int32_t (&c)
     for (int u = 0; u < U; u++)
       if (need & (1u << u)) {
         lo[u] = ps_load(a.xw + c[u]);
-        if constexpr (sizeof(T) == 8) hi[u] = ps_load(a.xw + a.n + c[u]);
+        if constexpr (sizeof(T) == 8) hi[u] = ps_load(a.xw + a.xn + c[u]);
       }
 #pragma unroll
     for (int u = 0; u < U; u++)
@@ -252,8 +254,9 @@ __device__ int ps_list_halo(const int32_t *__restrict__ ci, int nz, int64_t r0, 
   return total;
 }
 
+// Workgroup b of the sweep.
 template <typename T, int S, int Q>
-__global__ __launch_bounds__(PS_T) void ps_sweep_kernel(PsArgs<T> a) {
+__device__ __forceinline__ void ps_block(const PsArgs<T> &a, int b) {
   constexpr int R = 64 * Q, W = PS_W;
   constexpr int SP = S <= 4 ? 4 : (S <= 8 ? 8 : 16), LPC = 64 / SP;   // lanes that end with one column's sum
   constexpr int TPR = R > PS_T / 2 ? 1 : (R > PS_T / 4 ? 2 : (R > PS_T / 8 ? 4 : 8));
@@ -271,9 +274,8 @@ __global__ __launch_bounds__(PS_T) void ps_sweep_kernel(PsArgs<T> a) {
   uint16_t *scol = reinterpret_cast<uint16_t *>(hcol + a.hcap);   // [nzcap] columns as positions in [own rows | remote]
   uint32_t *bits = reinterpret_cast<uint32_t *>(smem_raw);   // set-up only, before sval and vh are filled
   const int t = threadIdx.x, lane = t & 63, w = __builtin_amdgcn_readfirstlane(t >> 6);
-  const int b = blockIdx.x;
-  const int64_t r0 = (int64_t)b * R;
-  const int rows = (int)min((int64_t)R, a.n - r0);
+  const int64_t r0 = a.n0 + (int64_t)b * R;
+  const int rows = (int)min((int64_t)R, a.n1 - r0);
   uint32_t tag = a.base;
   T *vp = va, *vn = vb;
 
@@ -417,15 +419,19 @@ __global__ __launch_bounds__(PS_T) void ps_sweep_kernel(PsArgs<T> a) {
         for (int s = 0; s < SP; s++) p[s] = s < S ? (double)(s * W + w == c ? self : acc[s < S ? s : 0]) : 0.0;
         const double d = wave_scatter<SP>(p, lane);
         const int sl = lane / LPC, col = sl * W + w;
-        if (lane % LPC == 0 && sl < S && col <= c)
-          ps_put(a.pw + (size_t)(2 * col) * a.G + b, a.pw + (size_t)(2 * col + 1) * a.G + b, d, tag);
+        if (lane % LPC == 0 && sl < S && col <= c) {
+          if (a.G == 1) s_dots[col] = d;     // nobody to exchange with
+          else ps_put(a.pw + (size_t)(2 * col) * a.G + b, a.pw + (size_t)(2 * col + 1) * a.G + b, d, tag);
+        }
         if (c >= S * W && w == W - 1) {      // no place for column c: the last one of a full basis
           const double sd = lanes_sum<64>((double)self);
-          if (lane == 0) ps_put(a.pw + (size_t)(2 * c) * a.G + b, a.pw + (size_t)(2 * c + 1) * a.G + b, sd, tag);
+          if (lane == 0 && a.G == 1) s_dots[c] = sd;
+          else if (lane == 0) ps_put(a.pw + (size_t)(2 * c) * a.G + b, a.pw + (size_t)(2 * c + 1) * a.G + b, sd, tag);
         }
       }
       bool ok = true;
-      if (w < PS_OWN) {
+      if (a.G == 1) {
+      } else if (w < PS_OWN) {
         // totals of the columns this workgroup adds: column b, b + G, ...; a
         // copy for each of 8 groups of workgroups, so that fewer poll one word
         for (int col = b + w * a.G; col <= c; col += PS_OWN * a.G) {
@@ -497,7 +503,7 @@ __global__ __launch_bounds__(PS_T) void ps_sweep_kernel(PsArgs<T> a) {
         vn[r] = v;
         if (st.done && r < rows) {
           if (c < a.c1 && !st.stop) {
-            if constexpr (sizeof(T) == 8) ps_put(a.xw + r0 + r, a.xw + a.n + r0 + r, v, tag);
+            if constexpr (sizeof(T) == 8) ps_put(a.xw + r0 + r, a.xw + a.xn + r0 + r, v, tag);
             else ps_store(a.xw + r0 + r, __builtin_bit_cast(uint32_t, v), tag);
           }
           a.V[(int64_t)c * a.ld + r0 + r] = v;
@@ -530,6 +536,28 @@ __global__ __launch_bounds__(PS_T) void ps_sweep_kernel(PsArgs<T> a) {
   }
 }
 
+template <typename T, int S, int Q>
+__global__ __launch_bounds__(PS_T) void ps_sweep_kernel(PsArgs<T> a) {
+  ps_block<T, S, Q>(a, blockIdx.x);
+}
+
+// Sweeps of several problems side by side, stacked row by row in one basis:
+// problem i has the workgroups b0 .. b0 + G - 1, its own columns, state,
+// coefficients and exchange words.
+template <typename T, int S, int Q>
+__global__ __launch_bounds__(PS_T) void ps_batch_kernel(PsArgs<T> a, const PsProb *__restrict__ probs,
+                                                        const int *__restrict__ of_block) {
+  const int i = of_block[blockIdx.x];
+  const PsProb p = probs[i];
+  a.n0 = p.n0; a.n1 = p.n1;
+  a.c0 = p.c0; a.c1 = p.c1; a.G = p.G;
+  a.pw += (size_t)2 * GS_MAXC * p.b0;
+  a.tw += (size_t)2 * PS_COPIES * GS_MAXC * i;
+  a.st += (size_t)GS_NSTATE * p.id;
+  a.dbuf += (size_t)a.dm * a.dm * p.id;
+  ps_block<T, S, Q>(a, blockIdx.x - p.b0);
+}
+
 // ---- admission: the sweeps in flight together must fit the CUs --------------
 // Workgroups go to the 8 XCDs in turn, so a sweep of G workgroups takes
 // ceil(G / 8) CUs of each; the budget is one XCD's CUs.
@@ -556,33 +584,46 @@ struct PsAdmit {
   }
 };
 
+// LDS of a workgroup's operator rows: its capacities in a, its bytes returned.
+// The rows' nonzeros with a quarter to spare (more than the room allows is
+// caught in the kernel), up to 4 remote entries per row in what they leave, a
+// quarter at least, and in the same memory at set-up two bits per column of
+// their span.
+template <typename T, int Q>
+size_t ps_lds(PsArgs<T> &a, size_t room, double nz_per_row, int64_t n) {
+  constexpr int R = 64 * Q;
+  const size_t nz = (size_t)(1.25 * nz_per_row * R) + 64;
+  const size_t left = room - std::min(nz * (sizeof(T) + 2), room - room / 4);
+  a.hcap = (int)std::min({(size_t)4 * R, (size_t)4096, left / (sizeof(T) + 4)}) & ~1;
+  const size_t rest = room - (size_t)a.hcap * (sizeof(T) + 4);
+  a.nzcap = (int)(std::min(nz, rest / (sizeof(T) + 2)) & ~(size_t)1);
+  const size_t span = ((size_t)n + 31) / 32 * 32;
+  a.wcap = (int)(std::min(span, (size_t)(a.nzcap + a.hcap) * sizeof(T) * 4) / 32 * 32);
+  return (size_t)a.nzcap * (sizeof(T) + 2) + (size_t)a.hcap * (sizeof(T) + 4);
+}
+
+// What the LDS leaves beside a kernel's static arrays, made available to it.
+template <typename T, int Q, typename K>
+int ps_room(K *kern, std::once_flag &once, hipError_t &err, size_t *room) {
+  constexpr int R = 64 * Q;
+  constexpr size_t fixed = sizeof(T) * (2 + PS_W) * R + 8 * GS_MAXC + 4 * (R + 1) + 1024;   // static LDS and slack
+  *room = (size_t)lds_max_bytes() - fixed;
+  std::call_once(once, [&] {
+    err = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)*room);
+  });
+  SA_HIP(err);
+  return 0;
+}
+
 template <typename T, int S, int Q>
 int ps_go(BV &V, const Mat *A, PsArgs<T> &a, hipStream_t s) {
   constexpr int R = 64 * Q;
   auto *kern = ps_sweep_kernel<T, S, Q>;
-  constexpr size_t fixed = sizeof(T) * (2 + PS_W) * R + 8 * GS_MAXC + 4 * (R + 1) + 1024;   // static LDS and slack
-  const size_t room = (size_t)lds_max_bytes() - fixed;
   static std::once_flag once;
   static hipError_t err = hipSuccess;
-  std::call_once(once, [&] {
-    err = hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)room);
-  });
-  SA_HIP(err);
-  size_t shm = 0;
-  if (A) {
-    // the rows' nonzeros with a quarter to spare (at least one more than the
-    // room allows is caught in the kernel), up to 4 remote entries per row, and
-    // in the same memory at set-up two bits per column of their span
-    // room / 4 at least goes to the remote entries, what the rows leave to them
-    const size_t nz = (size_t)(1.25 * (double)A->nnz / (double)std::max(1, A->n) * R) + 64;
-    const size_t left = room - std::min(nz * (sizeof(T) + 2), room - room / 4);
-    a.hcap = (int)std::min({(size_t)4 * R, (size_t)4096, left / (sizeof(T) + 4)}) & ~1;
-    const size_t rest = room - (size_t)a.hcap * (sizeof(T) + 4);
-    a.nzcap = (int)(std::min(nz, rest / (sizeof(T) + 2)) & ~(size_t)1);
-    shm = (size_t)a.nzcap * (sizeof(T) + 2) + (size_t)a.hcap * (sizeof(T) + 4);
-    const size_t span = ((size_t)V.n + 31) / 32 * 32;
-    a.wcap = (int)(std::min(span, (size_t)(a.nzcap + a.hcap) * sizeof(T) * 4) / 32 * 32);
-  }
+  size_t room, shm = 0;
+  SA_TRY((ps_room<T, Q>(kern, once, err, &room)));
+  if (A) shm = ps_lds<T, Q>(a, room, (double)A->nnz / (double)std::max(1, A->n), V.n);
   a.G = (int)((V.n + R - 1) / R);
   const int units = (a.G + N_XCD - 1) / N_XCD;
   PsAdmit admit(units);
@@ -645,7 +686,7 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
   const int q = ps_pick<T>(V.n, S, V.ps.share);
   if (!q) return 0;
   PsArgs<T> a{};
-  a.n = V.n; a.ld = V.ld; a.V = static_cast<T *>(V.data);
+  a.n0 = 0; a.n1 = a.xn = V.n; a.ld = V.ld; a.V = static_cast<T *>(V.data);
   if (A) { a.rp = A->rowptr; a.ci = A->col; a.val = static_cast<const T *>(A->val); }
   a.c0 = c0; a.c1 = c1;
   a.xw = V.ps.words;
@@ -678,6 +719,88 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
   return 0;
 }
 
+// ---- several problems at once -------------------------------------------------
+template <typename T, int S, int Q>
+int psb_go(const PsBatch &w, PsArgs<T> &a, int blocks, double nz_per_row, hipStream_t s) {
+  auto *kern = ps_batch_kernel<T, S, Q>;
+  static std::once_flag once;
+  static hipError_t err = hipSuccess;
+  size_t room;
+  SA_TRY((ps_room<T, Q>(kern, once, err, &room)));
+  const size_t shm = ps_lds<T, Q>(a, room, nz_per_row, a.xn);
+  PsAdmit admit((blocks + N_XCD - 1) / N_XCD);
+  hipLaunchKernelGGL(kern, dim3(blocks), dim3(PS_T), shm, s, a, (const PsProb *)w.probs, (const int *)w.of_block);
+  SA_HIP(hipGetLastError());
+  SA_HIP(hipStreamSynchronize(s));
+  return 0;
+}
+
+template <typename T, int S>
+int psb_rows(const PsBatch &w, PsArgs<T> &a, int q, int blocks, double nz, hipStream_t s) {
+  constexpr int M = sizeof(T) == 8 ? 88 : 176;
+  if constexpr (S * 22 <= M) if (q == 22) return psb_go<T, S, 22>(w, a, blocks, nz, s);
+  if constexpr (S * 16 <= M) if (q == 16) return psb_go<T, S, 16>(w, a, blocks, nz, s);
+  if constexpr (S * 11 <= M) if (q == 11) return psb_go<T, S, 11>(w, a, blocks, nz, s);
+  if (q == 8) return psb_go<T, S, 8>(w, a, blocks, nz, s);
+  return psb_go<T, S, 4>(w, a, blocks, nz, s);
+}
+
+template <typename T>
+int psb_run(PsBatch &w, PsArgs<T> &a, std::vector<PsProb> &pr, double nz_per_row, hipStream_t s, bool *done) {
+  constexpr int M = sizeof(T) == 8 ? 88 : 176;
+  const int most = std::min(num_cus(), 64 * PS_D);
+  int c1 = 0, len = 0;
+  int64_t nmax = 0;
+  for (const PsProb &p : pr) {
+    if (p.n1 <= p.n0 || p.c1 < p.c0) return 0;
+    c1 = std::max(c1, p.c1);
+    len = std::max(len, p.c1 - p.c0 + 1);
+    nmax = std::max(nmax, p.n1 - p.n0);
+  }
+  if (c1 > 64) return 0;
+  const int S = c1 <= 32 ? 4 : 8;
+  // as few rows per workgroup as lets all problems run in one launch; when
+  // none does, the most, and as many launches as that takes
+  int q = 0;
+  for (int t : {4, 8, 11, 16, 22}) {
+    if (S * t > M) break;
+    q = t;
+    int64_t total = 0;
+    for (const PsProb &p : pr) total += (p.n1 - p.n0 + 64 * q - 1) / (64 * q);
+    if (total <= most) break;
+  }
+  if ((nmax + 64 * q - 1) / (64 * q) > most) return 0;
+  const uint32_t tags = 4u * (uint32_t)len + 2u;
+  *w.fail = GsMirror{};
+  for (size_t i0 = 0; i0 < pr.size();) {
+    int blocks = 0;
+    size_t i1 = i0;
+    std::vector<int> of_block;
+    for (; i1 < pr.size(); i1++) {
+      PsProb &p = pr[i1];
+      p.G = (int)((p.n1 - p.n0 + 64 * q - 1) / (64 * q));
+      if (blocks + p.G > most) break;
+      p.b0 = blocks;
+      blocks += p.G;
+      of_block.insert(of_block.end(), p.G, (int)(i1 - i0));
+    }
+    if (w.tag > 0xffffffffu - tags) {
+      SA_HIP(hipMemsetAsync(w.words, 0, w.bytes, s));
+      w.tag = 1;
+    }
+    a.base = w.tag;
+    w.tag += tags;
+    // the copies have read their source when the launch below has been awaited
+    SA_HIP(hipMemcpyAsync(w.probs, pr.data() + i0, sizeof(PsProb) * (i1 - i0), hipMemcpyHostToDevice, s));
+    SA_HIP(hipMemcpyAsync(w.of_block, of_block.data(), sizeof(int) * blocks, hipMemcpyHostToDevice, s));
+    SA_TRY((S == 4 ? psb_rows<T, 4>(w, a, q, blocks, nz_per_row, s) : psb_rows<T, 8>(w, a, q, blocks, nz_per_row, s)));
+    if (w.fail->fail) return 0;
+    i0 = i1;
+  }
+  *done = true;
+  return 0;
+}
+
 }  // namespace
 
 size_t ps_bytes(int64_t n, int prec) {
@@ -690,6 +813,54 @@ int ps_sweep(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, boo
   *done = false;
   if (!V.ps.words || c1 >= GS_MAXC) return 0;
   return V.prec == SA_FP64 ? ps_run<double>(V, A, c0, c1, eta, s, done) : ps_run<float>(V, A, c0, c1, eta, s, done);
+}
+
+void ps_batch_free(PsBatch &w) {
+  if (w.words) (void)hipFree(w.words);
+  if (w.probs) (void)hipFree(w.probs);
+  if (w.of_block) (void)hipFree(w.of_block);
+  if (w.fail) (void)hipHostFree(w.fail);
+  w = PsBatch();
+}
+
+bool ps_batch_alloc(PsBatch &w, int64_t nrows, int prec, int P, hipStream_t s) {
+  if (w.words) return true;
+  // a launch has at most num_cus() workgroups, so no more problems
+  const int most = std::min(P, num_cus());
+  w.pw = (prec_size(prec) / 4) * (size_t)nrows;
+  w.tw = w.pw + (size_t)2 * GS_MAXC * num_cus();
+  w.abort_word = w.tw + (size_t)2 * PS_COPIES * GS_MAXC * most;
+  w.bytes = 8 * (w.abort_word + 1);
+  if (hipMalloc((void **)&w.words, w.bytes) != hipSuccess ||
+      hipMalloc((void **)&w.probs, sizeof(PsProb) * most) != hipSuccess ||
+      hipMalloc((void **)&w.of_block, sizeof(int) * num_cus()) != hipSuccess ||
+      hipHostMalloc((void **)&w.fail, sizeof(GsMirror)) != hipSuccess ||
+      hipMemsetAsync(w.words, 0, w.bytes, s) != hipSuccess) {
+    (void)hipGetLastError();
+    ps_batch_free(w);
+    return false;
+  }
+  w.tag = 1;
+  return true;
+}
+
+int ps_batch_sweep(PsBatch &w, int prec, void *V, int64_t ld, int64_t nrows, const int32_t *rp, const int32_t *ci,
+                   const void *val, int64_t nnz, std::vector<PsProb> &pr, GsState *st, double *dbuf, int m, double eta,
+                   hipStream_t s, bool *done) {
+  *done = false;
+  const double nz = nrows ? (double)nnz / (double)nrows : 0.0;
+  auto run = [&](auto zero) {
+    using T = decltype(zero);
+    PsArgs<T> a{};
+    a.xn = nrows; a.ld = ld; a.V = static_cast<T *>(V);
+    a.rp = rp; a.ci = ci; a.val = static_cast<const T *>(val);
+    a.xw = w.words; a.pw = w.words + w.pw; a.tw = w.words + w.tw;
+    a.abort_word = reinterpret_cast<unsigned int *>(w.words + w.abort_word);
+    a.st = st; a.host = w.fail; a.dbuf = dbuf; a.dm = m; a.eta = eta; a.refine = GS_REFINE_IFNEEDED;
+    a.polls = ps_polls();
+    return psb_run<T>(w, a, pr, nz, s, done);
+  };
+  return prec == SA_FP64 ? run(0.0) : run(0.0f);
 }
 
 }  // namespace sa

@@ -128,7 +128,7 @@ def coarse_modes(sa, theta, nmodes=NMODES, g=COARSE, tol=1e-6):
 
 def coarse_modes_batch(sa, thetas, nmodes=NMODES, g=COARSE, tol=1e-6, ncv=48):
     """The same eigenvectors for many parameter draws at once with the batched
-    solver (one workgroup per coarse problem, one launch per restart phase)."""
+    solver (workgroups of its own per coarse problem, one launch per restart phase)."""
     from .batch import Batch
     csrs = [sa.fv2d(g, g, th) for th in thetas]
     B = Batch(csrs)

@@ -45,6 +45,71 @@ def test_batched_matches_oracle(sa, orc, mixed, sweep):
     assert st["matvecs"] > 0 and (st["matvecs32"] > 0) == mixed
 
 
+def _chain(sa, n, seed):
+    """A symmetric tridiagonal matrix of n rows with a few separated ends."""
+    rng = np.random.default_rng(seed)
+    d = rng.uniform(1.0, 2.0, n)
+    d[rng.choice(n, min(n, 8), replace=False)] += 2.0 + np.arange(min(n, 8))
+    e = rng.uniform(0.1, 0.3, n - 1)
+    r = np.concatenate([np.arange(n), np.arange(n - 1), np.arange(1, n)])
+    c = np.concatenate([np.arange(n), np.arange(1, n), np.arange(n - 1)])
+    v = np.concatenate([d, e, e])
+    o = np.lexsort((c, r))
+    rp = np.zeros(n + 1, np.int32)
+    rp[1:] = np.cumsum(np.bincount(r, minlength=n))
+    return sa.CSR(n, rp, c[o].astype(np.int32), v[o])
+
+
+# rows of the problems, ncv, precision: one problem of a block and one of a row
+# more; all that one launch takes and more (256 workgroups); a basis of 32, 33
+# and 63 columns; rows that take every size of row block (4, 8, 11, 16, 22 chunks)
+RESIDENT = [
+    ([256], 24, False), ([257, 40, 1024, 1025], 32, False), ([300] * 256 + [290], 20, False),
+    ([511, 90, 64, 65], 33, True), ([4097, 130], 63, False), ([250000, 100], 16, False),
+    ([20000] * 9, 24, False), ([20000] * 17 + [33], 24, True)]
+
+
+@pytest.mark.parametrize("rows,ncv,mixed", RESIDENT)
+def test_batched_resident_sweep_edges(sa, rows, ncv, mixed):
+    """The resident sweep and the lock-step one give the same eigenvalues (both
+    have converged to the tolerance) and error estimates below it."""
+    from slepc_amd.batch import Batch
+    csrs = [_chain(sa, n, 7 + i % 5) for i, n in enumerate(rows)]
+    out = []
+    for sweep in ("persistent", "wide"):
+        B = Batch(csrs)
+        B.set_sweep(sweep)
+        B.solve(4, ncv, 1e-10, "LM", mixed=mixed)
+        assert B.sweep_info()["mode"] == sweep
+        assert all(B.converged(p)[2] == 1 for p in range(len(rows)))
+        assert np.all(B.errors() <= 1e-10)
+        out.append(np.array([[B.eigenpair(p, i, False)[0] for i in range(4)] for p in range(len(rows))]))
+    assert np.allclose(out[0], out[1], rtol=1e-10, atol=0)
+
+
+GIVE_UP = """
+import sys, numpy as np
+sys.path.insert(0, %r)
+sys.path.insert(0, %r)
+import slepc_amd as sa
+import test_gpu_batched as t
+sa.init(0)
+t.test_batched_resident_sweep_edges(sa, [2000, 300, 5000], 24, False)
+t.test_batched_resident_sweep_edges(sa, [2000, 300, 5000], 24, True)
+"""
+
+
+def test_batched_resident_sweep_gives_up():
+    """With no polls allowed the resident sweep gives up half-way and the
+    lock-step sweep starts over: the same results."""
+    import os
+    import subprocess
+    import sys
+    here = os.path.dirname(os.path.abspath(__file__))
+    env = dict(os.environ, SLEPC_AMD_SWEEP_POLLS="0")
+    subprocess.run([sys.executable, "-c", GIVE_UP % (os.path.dirname(here), here)], check=True, env=env, timeout=100)
+
+
 @pytest.mark.parametrize("P", [1, 7, 8, 9, 33])
 def test_batched_projected_problems_on_host_threads(sa, orc, P):
     """From 8 problems on the projected problems go to the solve's own host

@@ -40,10 +40,12 @@
 // tile with two shuffle reductions per step (up to 32 columns) and one thread per
 // row (beyond), 2.1M rows FP64: 8 columns 314 -> 238 us, 16: 721 -> 523, 24: 2.04 ->
 // 0.95 ms, 32: 2.75 -> 1.47, 48: 13.0 -> 4.9, 64: 16.9 -> 7.2 (floor of 32 columns at
-// the copy rate: 0.23 ms).
+// the copy rate: 0.45 ms, V read and written twice).  Forming Q by matrix products
+// (tsqr_form_kernel) then took 32 columns to 1.30 ms.
 #include <algorithm>
 #include <cmath>
 #include <cstdint>
+#include <mutex>
 #include <vector>
 
 #include "sa_device.h"
@@ -207,18 +209,14 @@ __global__ __launch_bounds__(64 * W) void tsqr_factor_kernel(const T *A, int64_t
                                  sh);
 }
 
-// Q of one tree level: tile b applies its reflectors (rows x k Y in geqrf
-// layout, scalars tau[b k ..]) in descending order to [C_b; 0], C_b = rows b k
-// .. b k + k - 1 of the Q of the level above (ldc), which gives its rows of Q;
-// with C == nullptr (the top tile) to [I; 0], the explicit Householder factor
-// (dorg2r).  The result, times sgn[c] per column when sgn is given, goes to
-// out (may equal Y: each lane reads only its own rows of Y, those of step j - 1
-// one step ahead).
+// Q of one tree level, reflector by reflector (up to 8 columns; what it computes
+// is said at tsqr_form_kernel).  Each lane reads only its own rows of Y, those of
+// step j - 1 one step ahead, so out may equal Y.
 template <typename T, int K, int RPL, int W>
-__global__ __launch_bounds__(64 * W) void tsqr_form_kernel(const T *Y, int64_t ldy, int64_t rows, int k,
-                                                                        const T *__restrict__ tau,
-                                                                        const T *__restrict__ C, int64_t ldc, T *out,
-                                                                        int64_t ldo, const T *__restrict__ sgn) {
+__global__ __launch_bounds__(64 * W) void tsqr_form_steps_kernel(const T *Y, int64_t ldy, int64_t rows, int k,
+                                                                 const T *__restrict__ tau, const T *__restrict__ C,
+                                                                 int64_t ldc, T *out, int64_t ldo,
+                                                                 const T *__restrict__ sgn) {
   constexpr int TR = 64 * RPL * W, SP = ts_pow2(K), LPC = 64 / SP;
   __shared__ TsShared<T, K, W> sh;
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -283,6 +281,199 @@ __global__ __launch_bounds__(64 * W) void tsqr_form_kernel(const T *Y, int64_t l
   }
 }
 
+// Shared memory of tsqr_form_kernel: the tile's Gram matrix beside what its
+// phases use in turn.
+template <typename T, int K, int W>
+struct TsForm {
+  static constexpr int NB = (K + 15) / 16, KP = 16 * NB, LD = KP + 1, NBLK = NB * (NB + 1) / 2;
+  T G[KP * LD];                        // (Y^T Y)(j, i) at G[j LD + i], j < i
+  T tau[KP];
+  union {
+    T tr[W][KP * 17];                  // 16 rows of a wave, transposed
+    T sum[(W + 1) / 2][NBLK * 256];    // Gram blocks on their way to wave 0
+    struct {
+      T X[KP * LD], Y1[KP * LD], C[KP * LD];   // row by row
+    } s;
+  };
+};
+
+// Q of one tree level: tile b applies its reflectors (rows x k Y in geqrf
+// layout, scalars tau[b k ..]) in descending order to [C_b; 0], C_b = rows b k
+// .. b k + k - 1 of the Q of the level above (ldc), which gives its rows of Q;
+// with C == nullptr (the top tile) to [I; 0], the explicit Householder factor
+// (dorg2r).  The result, times sgn[c] per column when sgn is given, goes to
+// out (may equal Y: a workgroup reads its whole tile before it writes).
+//
+// The reflectors are applied together (compact WY form; Schreiber and Van Loan,
+// SIAM J. Sci. Stat. Comput. 10, 1989): Q = [C; 0] - Y X, where row j of X is
+// what reflector j would subtract, x_j = tau_j (y_j^T [C; 0] - sum_{i > j}
+// (y_j^T y_i) x_i).  The tile's rows are read once into registers, lane l holding
+// row l % 16 and column l / 16 of each 16 x 4 block; Y^T Y (through a transpose
+// in LDS) and Y X are matrix products on the MFMA units and what is left, k x k
+// per tile, is a triangular solve.  Memory bounds it (the level over V of 2.1M
+// rows and 32 columns FP64 takes 386 us, 226 at the copy rate), then the solve,
+// which only the two tiles a CU holds overlap.  Against applying the
+// reflectors one by one, each a reduction and an update of all columns (the
+// whole factorization, 2.1M rows FP64): 16 columns 523 -> 481 us, 24 950 -> 874,
+// 32 1471 -> 1301, 48 4.9 -> 3.4 ms, 64 7.2 -> 5.0; 8 columns, which the matrix units
+// pad to 16, 238 -> 260, so they keep the steps.  Eight waves per tile have the
+// shorter phases; with 32 columns FP64 they lose to four (1375 us).
+template <typename T, int K, int RPL, int W>
+__global__ __launch_bounds__(64 * W) void tsqr_form_kernel(const T *Y, int64_t ldy, int64_t rows, int k,
+                                                           const T *__restrict__ tau, const T *__restrict__ C,
+                                                           int64_t ldc, T *out, int64_t ldo,
+                                                           const T *__restrict__ sgn) {
+  using F = TsForm<T, K, W>;
+  using V4 = typename Vec4<T>::type;
+  constexpr int TR = 64 * RPL * W, NB = F::NB, KP = F::KP, LD = F::LD, NBLK = F::NBLK;
+  constexpr int RB = 4 * RPL, NU = (K + 3) / 4, NT = 64 * W;   // 16-row blocks per wave, 4-column steps
+  extern __shared__ __align__(16) unsigned char ts_raw[];
+  F &sh = *reinterpret_cast<F *>(ts_raw);
+  const int t = threadIdx.x, lane = t & 63, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int g = lane >> 4, c16 = lane & 15;
+  const int64_t b = blockIdx.x;
+  const int64_t r0 = b * TR;
+  const int nb = (int)min((int64_t)TR, rows - r0);
+  const int kk = min(k, nb);                    // rows of C_b beyond the tile's rows meet zero rows of its R
+  T y[RB][NU];
+#pragma unroll
+  for (int rb = 0; rb < RB; rb++) {
+    const int row = 16 * (wv * RB + rb) + c16;
+#pragma unroll
+    for (int u = 0; u < NU; u++) {
+      const int c = 4 * u + g;
+      y[rb][u] = (c < kk && row < nb) ? Y[r0 + row + (int64_t)c * ldy] : (T)0;
+    }
+  }
+  constexpr int NC = (KP * KP + NT - 1) / NT;
+  T cv[NC];                                     // C_b, on its way to LDS
+#pragma unroll
+  for (int i = 0; i < NC; i++) {
+    const int r = (t + i * NT) % KP, c = (t + i * NT) / KP;
+    if (C) cv[i] = (r < kk && c < k) ? C[b * k + r + (int64_t)c * ldc] : (T)0;
+    else cv[i] = (r == c && r < kk) ? (T)1 : (T)0;
+  }
+  for (int i = t; i < KP; i += NT) sh.tau[i] = i < kk ? tau[b * k + i] : (T)0;
+  if (wv == 0) {                                // unit lower trapezoidal: R is above
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+      for (int u = 0; u < NU; u++) {
+        const int row = 16 * rb + c16, c = 4 * u + g;
+        y[rb][u] = row > c ? y[rb][u] : ((row == c && c < kk) ? (T)1 : (T)0);
+      }
+  }
+  // ---- G = Y^T Y, the blocks on and above the diagonal -----------------------
+  V4 acc[NBLK];
+#pragma unroll
+  for (int q = 0; q < NBLK; q++) acc[q] = (V4){0, 0, 0, 0};
+  T *tr = sh.tr[wv];
+#pragma unroll
+  for (int rb = 0; rb < RB; rb++) {
+#pragma unroll
+    for (int u = 0; u < NU; u++) tr[(4 * u + g) * 17 + c16] = y[rb][u];
+#pragma unroll
+    for (int h = 0; h < 4; h++) {
+      T a[NB];
+#pragma unroll
+      for (int q = 0; q < NB; q++) a[q] = 16 * q + c16 < 4 * NU ? tr[(16 * q + c16) * 17 + 4 * h + g] : (T)0;
+      int at = 0;
+#pragma unroll
+      for (int q = 0; q < NB; q++)
+#pragma unroll
+        for (int p = q; p < NB; p++, at++) acc[at] = mfma16x16x4(a[q], a[p], acc[at]);
+    }
+  }
+  // waves in pairs, the same order every time
+#pragma unroll
+  for (int half = W / 2; half >= 1; half /= 2) {
+    __syncthreads();
+    if (wv >= half && wv < 2 * half) {
+#pragma unroll
+      for (int q = 0; q < NBLK; q++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) sh.sum[wv - half][q * 256 + v * 64 + lane] = acc[q][v];
+    }
+    __syncthreads();
+    if (wv < half) {
+#pragma unroll
+      for (int q = 0; q < NBLK; q++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) acc[q][v] += sh.sum[wv][q * 256 + v * 64 + lane];
+    }
+  }
+  __syncthreads();
+  if (wv == 0) {
+    int at = 0;
+#pragma unroll
+    for (int q = 0; q < NB; q++)
+#pragma unroll
+      for (int p = q; p < NB; p++, at++)
+#pragma unroll
+        for (int v = 0; v < 4; v++) sh.G[(16 * q + mfma_row<T>(g, v)) * LD + 16 * p + c16] = acc[at][v];
+#pragma unroll
+    for (int rb = 0; rb < NB; rb++)
+#pragma unroll
+      for (int u = 0; u < NU; u++) sh.s.Y1[(16 * rb + c16) * LD + 4 * u + g] = y[rb][u];
+  }
+#pragma unroll
+  for (int i = 0; i < NC; i++) {
+    const int r = (t + i * NT) % KP, c = (t + i * NT) / KP;
+    if (c < KP) sh.s.C[r * LD + c] = cv[i];
+  }
+  __syncthreads();
+  // ---- X, 16 rows at a time from the last -------------------------------------
+#pragma unroll
+  for (int q = NB - 1; q >= 0; q--) {
+    for (int e = t; e < 16 * KP; e += NT) {
+      const int j = 16 * q + e / KP, c = e % KP;
+      T s = (T)0;
+      if (j < 4 * NU) {
+#pragma unroll 8
+        for (int r = 16 * q; r < KP; r++) s += sh.s.Y1[r * LD + j] * sh.s.C[r * LD + c];
+#pragma unroll 8
+        for (int i = 16 * (q + 1); i < KP; i++) s -= sh.G[j * LD + i] * sh.s.X[i * LD + c];
+      }
+      sh.s.X[j * LD + c] = s;
+    }
+    __syncthreads();
+    if (t < KP) {
+      T x[16];
+#pragma unroll
+      for (int j = 15; j >= 0; j--) {
+        T s = sh.s.X[(16 * q + j) * LD + t];
+#pragma unroll
+        for (int i = 15; i > j; i--) s -= sh.G[(16 * q + j) * LD + 16 * q + i] * x[i];
+        x[j] = sh.tau[16 * q + j] * s;
+        sh.s.X[(16 * q + j) * LD + t] = x[j];
+      }
+    }
+    __syncthreads();
+  }
+  // ---- Q = [C; 0] - Y X ---------------------------------------------------------
+#pragma unroll
+  for (int q = 0; q < NB; q++) {
+    T xa[NU];
+#pragma unroll
+    for (int u = 0; u < NU; u++) xa[u] = sh.s.X[(4 * u + g) * LD + 16 * q + c16];
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++) {
+      V4 d = (V4){0, 0, 0, 0};
+#pragma unroll
+      for (int u = 0; u < NU; u++) d = mfma16x16x4(xa[u], y[rb][u], d);
+      const int row = 16 * (wv * RB + rb) + c16;
+#pragma unroll
+      for (int v = 0; v < 4; v++) {
+        const int c = 16 * q + mfma_row<T>(g, v);
+        if (row < nb && c < k) {
+          T o = row < KP ? sh.s.C[row * LD + c] - d[v] : -d[v];
+          out[r0 + row + (int64_t)c * ldo] = sgn ? o * sgn[c] : o;
+        }
+      }
+    }
+  }
+}
+
 // ---- host side ----------------------------------------------------------------
 
 void tsqr_signs(const double *Qtop, const double *R, int64_t n, int k, double *f) {
@@ -325,13 +516,27 @@ struct TsLevel {
 template <typename T, int K>
 int tsqr_t(BV &V, int l, int k, bool formq, double *R_host, double *f, hipStream_t s) {
   constexpr int RPL = K <= 16 ? 4 : (K <= 32 ? 2 : 1), WV = K <= 32 ? 4 : 8, TR = 64 * RPL * WV;
+  constexpr int WF = K == 32 && sizeof(T) == 8 ? 4 : 8;   // waves of a tile whose Q is formed
   auto factor = [&](const T *A, int64_t lda, int64_t rows, int G, T *Y, int64_t ldy, T *tau, T *R, int64_t ldr) {
     tsqr_factor_kernel<T, K, RPL, WV><<<G, 64 * WV, 0, s>>>(A, lda, rows, k - l, Y, ldy, tau, R, ldr);
   };
   auto form = [&](const T *Y, int64_t ldy, int64_t rows, int G, const T *tau, const T *C, int64_t ldc, T *out,
                   int64_t ldo, const T *sg) {
-    tsqr_form_kernel<T, K, RPL, WV><<<G, 64 * WV, 0, s>>>(Y, ldy, rows, k - l, tau, C, ldc, out, ldo, sg);
+    if constexpr (K <= 8)
+      tsqr_form_steps_kernel<T, K, RPL, WV><<<G, 64 * WV, 0, s>>>(Y, ldy, rows, k - l, tau, C, ldc, out, ldo, sg);
+    else
+      tsqr_form_kernel<T, K, TR / (64 * WF), WF><<<G, 64 * WF, sizeof(TsForm<T, K, WF>), s>>>(Y, ldy, rows, k - l, tau,
+                                                                                           C, ldc, out, ldo, sg);
   };
+  if constexpr (K > 8) {
+    static std::once_flag once;
+    static hipError_t err = hipSuccess;
+    std::call_once(once, [] {
+      err = hipFuncSetAttribute((const void *)tsqr_form_kernel<T, K, TR / (64 * WF), WF>,
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(TsForm<T, K, WF>));
+    });
+    SA_HIP(err);
+  }
   const int nk = k - l;
   const int64_t n = V.n;
   // level sizes: rows_{i+1} = tiles_i * nk until one tile is left

@@ -80,8 +80,8 @@ A64_nnz = [0]
 
 
 def sweep_roofline(sa, A64, n, m):
-    """One m-step Arnoldi sweep (fused SpMV + CGS + DGKS kernels and their
-    one-workgroup reductions only), timed with HIP events on the library
+    """One m-step Arnoldi sweep (the resident kernel, or SpMV, Gram-Schmidt
+    slots and their one-workgroup reductions only), timed with HIP events on the library
     stream.  Algorithmic bytes: per step the SpMV (values, indices, row
     pointers, x, y) and per Gram-Schmidt pass 2(c+1) basis columns (dots read
     c columns, the update reads c columns and v and writes v)."""
@@ -492,15 +492,15 @@ def main():
               "cpu_oracle_seconds_1_thread": round(r1s["seconds"], 4), "cpu_oracle_restarts": r1["its"]}
         log("c1: %s" % json.dumps(c1))
 
-    # ---------------- roofline of the fused Gram-Schmidt kernels
+    # ---------------- roofline of the Arnoldi sweep kernels
     A64_nnz[0] = probs[0][1].nnz
     gbs, tot_bytes, ms, passes = sweep_roofline(sa, probs[0][2], n, NCV)
     roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": profiled_traffic("fv2d_256"),
-            "kernel": "gs_kernel + gs_sum_kernel (fused SpMV + CGS + DGKS), one launch unit = one 64-step sweep",
+            "kernel": "ps_sweep_kernel (resident SpMV + CGS + DGKS), one launch = one 64-step sweep",
             "note": "64-step Arnoldi sweep on the headline operator (n=65,536, %.2f passes/step): %.1f MB "
-                    "algorithmic in %.3f ms (HIP events); the 34 MB basis stays cache-resident and each kernel "
-                    "is a few microseconds, so latency bounds it; traffic = counter-measured HBM bytes per sweep "
+                    "algorithmic in %.3f ms (HIP events); the 34 MB basis stays in registers and the exchanges between "
+                    "workgroups (about 1.3 us each, five per step) bound it; traffic = counter-measured HBM bytes per sweep "
                     "from profiles/gs_sweep_fv2d_256.txt" % (passes, tot_bytes / 1e6, ms)}
 
     roof["spmv_fv2d_256"] = spmv_roofline(sa, probs[0][1])

@@ -498,7 +498,7 @@ int sa_eps_get_stats(sa_eps eps, sa_eps_stats *st);
  * Each problem runs the default Krylov-Schur of krylovschur.c:227-348 (Lanczos
  * + DSHEP, locking, keep 0.5) on its own; all problems share one block-diagonal
  * operator and one basis in HBM, and one restart phase of every problem is one
- * kernel launch (a workgroup per problem).  No counterpart type in the
+ * kernel launch (workgroups of its own for each).  No counterpart type in the
  * reference: it is the drop-in for a loop of EPSSolve calls over the problems.
  * Input: P problems, n[p] rows each; rowptr holds the P local row-pointer
  * arrays (n[p]+1 entries each) back to back, col/val the P local CSR arrays. */
@@ -526,20 +526,20 @@ int sa_batch_compute_errors(sa_batch batch, int nev, double *err);
 int sa_batch_get_stats(sa_batch batch, int64_t *counters6, double *seconds3);
 /* Sweep kernel of the batch: 0 autotune (default; both are timed on the first
    restart round of the first solve phase of each precision and basis width,
-   and the faster is kept for later solves of the batch), 1 one workgroup
-   per problem runs the whole sweep (ncv < 64), 2 lock-step: each Gram-Schmidt
+   and the faster is kept for later solves of the batch), 1 resident: every
+   problem's basis in the registers of its own workgroups (ncv < 64), 2 lock-step: each Gram-Schmidt
    slot of every active problem is one launch over all their 64-row chunks.
    The getter returns the mode used by the last FP64 phase and the autotuner's
    timings of one sweep (milliseconds, -1 when not timed). */
 int sa_batch_set_sweep(sa_batch batch, int mode);
 int sa_batch_get_sweep(sa_batch batch, int *mode, double *ms_persistent, double *ms_wide);
 /* The schedule autotuner (mode 0) times, on the first restart round, the
-   one-workgroup sweep (when ncv < 64) and three lock-step tile schedules:
+   resident sweep (when ncv < 64) and three lock-step tile schedules:
    the default (non-temporal tile loads for a basis above 256 MiB, SpMV lanes
    per row from the mean row length), the other tile-load kind, and twice the
    lanes; it reruns the fastest so the round's results are its own.  The
-   getter returns the last solve's schedule (kind 1 one workgroup per
-   problem, 2 lock-step; nt; lanes) and the four timings in milliseconds (-1:
+   getter returns the last solve's schedule (kind 1 resident,
+   2 lock-step; nt; lanes) and the four timings in milliseconds (-1:
    not timed).  No counterpart in the reference. */
 int sa_batch_get_schedule(sa_batch batch, int *kind, int *nt, int *lanes, double *ms4);
 /* Lock-step restart sweeps replayed from HIP graphs (default on): each sweep

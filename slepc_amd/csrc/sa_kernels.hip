@@ -311,7 +311,7 @@ int launch_multvec(BV &V, int l, int k, double alpha, const double *q_dev, doubl
 // multinplace_kernel (for Q slices too large for LDS): a workgroup owns 64
 // rows, stages V(rows, l:k) in LDS, then each wave computes a 16-row slab of
 // the output with 16x16x4 MFMA tiles, reading Q from global memory.  The
-// Q-in-LDS kernel below is the common path (2.6x faster at 2.1M rows).
+// Q-in-LDS kernel below is the common path (2.6x faster when it came, 2.1M rows).
 // ---------------------------------------------------------------------------
 constexpr int MIP_NT = 8;   // up to 8 output tiles of 16 columns (128 columns)
 
@@ -485,7 +485,8 @@ __global__ __launch_bounds__(BLK) void multinplace_q_kernel(int64_t n, int64_t l
 template <typename T, int NTL, int VL>
 static void launch_mip_rows(BV &V, int l, int K, int s_, int N, const double *Q_dev, int ldq, hipStream_t s) {
   const int64_t rows = 4 * 16 * VL;                // per workgroup step
-  const int grid = (int)std::min<int64_t>((V.n + rows - 1) / rows, VL == 1 ? MIP_GRID : (NTL == 1 ? 3 * MIP_GRID / 2 : MIP_GRID / 2));
+  const int most = VL == 1 ? MIP_GRID : (NTL == 1 ? 3 * MIP_GRID / 2 : MIP_GRID / 2);
+  const int grid = (int)std::min<int64_t>((V.n + rows - 1) / rows, most);
   const size_t shm = (size_t)((K + 3) & ~3) * (NTL * 16 + 1) * sizeof(T);
   if (V.n * (int64_t)K * (int64_t)sizeof(T) > GS_NT_BYTES)
     hipLaunchKernelGGL((multinplace_q_kernel<T, NTL, VL, true>), dim3(grid), dim3(BLK), shm, s, V.n, V.ld,

@@ -500,12 +500,14 @@ template <typename T, int NTL>
 static void launch_mip_q(BV &V, int l, int K, int s_, int N, const double *Q_dev, int ldq, hipStream_t s) {
   constexpr int VL = 16 / (int)sizeof(T);
   // 16 bytes per lane, or one row per lane for few output columns and on small
-  // blocks, where more waves count (microseconds with 16 bytes and with one row, FP64:
-  // K = 30, N = 15 at 1.5M rows 106.8, 108.3, K = 20, N = 10 at 300,000 32.8, 30.4; K = 32,
-  // N = 16 at 30,000 23.6, 22.1; K = 90, N = 48 at 50,000 50.9, 52.1, at 100,000 61.6,
-  // 66.6; FP32 four rows per lane: at 100,000 53.2, 50.4)
-  constexpr int shift = sizeof(T) == 8 ? (NTL > 1 ? 22 : 25) : (NTL > 1 ? 24 : 62);
-  if (V.n * K >= (int64_t)1 << shift) launch_mip_rows<T, NTL, VL>(V, l, K, s_, N, Q_dev, ldq, s);
+  // blocks, where more waves count (microseconds with 16 bytes and with one row,
+  // FP64: K = 30, N = 15 at 1.5M rows 106.8, 108.3, K = 20, N = 10 at 300,000 32.8, 30.4;
+  // K = 61, N = 34 at 159,556 57.7, 57.5, K = 40, N = 20 at 250,000 45.6, 44.0, K = 61,
+  // N = 33 at 180,000 56.4, 57.4, K = 64, N = 48 at 200,000 66.8, 69.9, K = 80, N = 40 at
+  // 400,000 104.6, 116.6; FP32 four rows per lane: at 100,000 53.2, 50.4)
+  constexpr int64_t M = (int64_t)1 << 20, from = sizeof(T) == 8 ? (NTL > 1 ? 10 * M : 32 * M) : 16 * M;
+  constexpr bool wide = sizeof(T) == 8 || NTL > 1;
+  if (wide && V.n * K >= from) launch_mip_rows<T, NTL, VL>(V, l, K, s_, N, Q_dev, ldq, s);
   else launch_mip_rows<T, NTL, 1>(V, l, K, s_, N, Q_dev, ldq, s);
 }
 

@@ -7,8 +7,9 @@
 // w + 8, ...: a chunk is up to NC loads per lane, those of the next chunk in
 // flight while the current one is used.  The update v - V h needs one sum over
 // the waves per chunk (LDS, one barrier that leaves the loads in flight); the
-// dot products accumulate in FP64 registers and meet in one wave reduction at
-// the end.
+// dot products accumulate in FP64 registers, FP32 products too one by one (as
+// many instructions as FP32 pairs that are then converted: the same time), and
+// meet in one wave reduction at the end.
 //
 // HBM bounds it: the basis is read three times per two-pass step, and a slot
 // reads 6.2 TB/s at 57 columns of 2.1M FP64 rows (949 MB in 152 us).  The
@@ -110,17 +111,13 @@ __device__ __forceinline__ void gw_rows(const GsArgs<T> &a, int64_t first, int64
       }
     }
     if constexpr (DOTS) {
-      T s = (T)0;
 #pragma unroll
-      for (int e = 0; e < VL; e++) s += v[e] * v[e];
-      self += (double)s;
+      for (int e = 0; e < VL; e++) self += (double)v[e] * (double)v[e];
 #pragma unroll
       for (int i = 0; i < NC; i++)
         if (i * GW_W + w < c) {
-          T d = (T)0;
 #pragma unroll
-          for (int e = 0; e < VL; e++) d += x[i][e] * v[e];
-          acc[i] += (double)d;
+          for (int e = 0; e < VL; e++) acc[i] += (double)x[i][e] * (double)v[e];
         }
     }
   }

@@ -254,6 +254,45 @@ __device__ int ps_list_halo(const int32_t *__restrict__ ci, int nz, int64_t r0, 
   return total;
 }
 
+// The lane's products of v with the first N column slots, and of v with itself,
+// added to acc and self: sums of RUN rows in T, those in FP64.  Long FP32 sums
+// would be the larger part of a coefficient's error: with all 22 rows of a lane
+// in one, coefficients against 10 columns of 354,000 rows were 4.5e-10 of the
+// vector's norm off and the norm 3.1e-10; sums as short as those of 256 threads
+// on a 64-row tile (3 rows for 10 columns, 10 for 32, 11 for 40, 22 for 64) leave
+// 1.8e-10 and 5.5e-11.  So FP32 products against up to 32 or 40 columns are added in
+// FP64 one by one, beyond in runs of 8, with more than 64 columns of 11 at most.
+template <int N, int RUN, typename T, int S, int Q>
+__device__ __forceinline__ void ps_dots(T (&x)[S][Q], const T *vn, int lane, double (&acc)[S], double &self) {
+#pragma unroll
+  for (int q0 = 0; q0 < Q; q0 += RUN) {
+    T part[N], sq = (T)0;
+#pragma unroll
+    for (int s = 0; s < N; s++) part[s] = (T)0;
+#pragma unroll
+    for (int q = q0; q < Q && q < q0 + RUN; q++) {
+      const T v = vn[q * 64 + lane];
+      if constexpr (RUN == 1) {
+        self += (double)v * (double)v;
+#pragma unroll
+        for (int s = 0; s < N; s++) {
+          asm volatile("" : "+v"(x[s][q]));      // converted here, not kept as doubles
+          acc[s] += (double)x[s][q] * (double)v;
+        }
+      } else {
+        sq += v * v;
+#pragma unroll
+        for (int s = 0; s < N; s++) part[s] += x[s][q] * v;
+      }
+    }
+    if constexpr (RUN > 1) {
+      self += (double)sq;
+#pragma unroll
+      for (int s = 0; s < N; s++) acc[s] += (double)part[s];
+    }
+  }
+}
+
 // Workgroup b of the sweep.
 template <typename T, int S, int Q>
 __device__ __forceinline__ void ps_block(const PsArgs<T> &a, int b) {
@@ -261,6 +300,7 @@ __device__ __forceinline__ void ps_block(const PsArgs<T> &a, int b) {
   constexpr int SP = S <= 4 ? 4 : (S <= 8 ? 8 : 16), LPC = 64 / SP;   // lanes that end with one column's sum
   constexpr int TPR = R > PS_T / 2 ? 1 : (R > PS_T / 4 ? 2 : (R > PS_T / 8 ? 4 : 8));
   constexpr int U = 4;                       // nonzeros in flight per thread
+  constexpr int NS = S > 8 ? 5 : 4;          // FP32: column slots up to which products are added in FP64
   __shared__ T va[R], vb[R];                 // the last column and the one being computed
   __shared__ T red[W * R];
   __shared__ double s_dots[GS_MAXC];
@@ -404,19 +444,14 @@ __device__ __forceinline__ void ps_block(const PsArgs<T> &a, int b) {
       // partial dot products of the block, and its sum of squares in the place
       // of column c (held by no wave yet)
       {
-        double p[SP];
-        T acc[S], self = (T)0;
+        double p[SP], acc[S], self = 0.0;
 #pragma unroll
-        for (int s = 0; s < S; s++) acc[s] = (T)0;
+        for (int s = 0; s < S; s++) acc[s] = 0.0;
+        if constexpr (sizeof(T) == 8) ps_dots<S, Q>(x, vn, lane, acc, self);
+        else if (c < NS * W) ps_dots<NS, 1>(x, vn, lane, acc, self);
+        else ps_dots<S, (S > 8 ? Q : 8)>(x, vn, lane, acc, self);
 #pragma unroll
-        for (int q = 0; q < Q; q++) {
-          const T v = vn[q * 64 + lane];
-          self += v * v;
-#pragma unroll
-          for (int s = 0; s < S; s++) acc[s] += x[s][q] * v;
-        }
-#pragma unroll
-        for (int s = 0; s < SP; s++) p[s] = s < S ? (double)(s * W + w == c ? self : acc[s < S ? s : 0]) : 0.0;
+        for (int s = 0; s < SP; s++) p[s] = s < S ? (s * W + w == c ? self : acc[s < S ? s : 0]) : 0.0;
         const double d = wave_scatter<SP>(p, lane);
         const int sl = lane / LPC, col = sl * W + w;
         if (lane % LPC == 0 && sl < S && col <= c) {
@@ -424,7 +459,7 @@ __device__ __forceinline__ void ps_block(const PsArgs<T> &a, int b) {
           else ps_put(a.pw + (size_t)(2 * col) * a.G + b, a.pw + (size_t)(2 * col + 1) * a.G + b, d, tag);
         }
         if (c >= S * W && w == W - 1) {      // no place for column c: the last one of a full basis
-          const double sd = lanes_sum<64>((double)self);
+          const double sd = lanes_sum<64>(self);
           if (lane == 0 && a.G == 1) s_dots[c] = sd;
           else if (lane == 0) ps_put(a.pw + (size_t)(2 * c) * a.G + b, a.pw + (size_t)(2 * c + 1) * a.G + b, sd, tag);
         }

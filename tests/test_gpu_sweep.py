@@ -157,3 +157,28 @@ def test_sweep_gives_up_and_starts_over(tmp_path):
     assert np.abs(a["V"] - b["V"]).max() <= 1e-12
     assert np.abs(a["H"] - b["H"]).max() <= 1e-13
     assert float(a["nrm"]) == pytest.approx(float(b["nrm"]), rel=1e-14)
+
+
+# up to 32 columns of the resident sweep, one row and 22 rows per lane; the
+# streaming slots at any width
+@pytest.mark.parametrize("n,j", [(65, 7), (354000, 1), (354000, 10), (354000, 31), (400001, 2), (400001, 60),
+                                 (370001, 110)])
+def test_fp32_products_are_added_in_fp64(sa, n, j):
+    """Orthonormalising an FP32 column: coefficients and norm equal those of the
+    stored values in FP64.  A product of two FP32 numbers is exact in FP64 and
+    a sum of FP64 is at most 40 additions deep on either side, so the two differ
+    by at most 80 eps of ||x|| ||v||; FP32 sums of a few rows are 1e-10 off at
+    these sizes."""
+    rng = np.random.default_rng(n + j)
+    V = sa.BV(n, j + 1, sa.FP32)
+    B = np.linalg.qr(rng.standard_normal((n, j)))[0]
+    for i in range(j):
+        V.set_column(i, B[:, i])
+    V.set_column(j, rng.standard_normal(n))
+    X, v = V.get_matrix(j), V.get_column(j)      # as stored
+    nrm, lindep = V.orthonormalize_column(j)
+    H = V.coefficients(j, j + 1)[:, 0]
+    ref, h = np.linalg.norm(v), X.T @ v
+    assert not lindep
+    assert np.abs(H[:j] - h).max() <= 80 * EPS["fp64"] * ref
+    assert nrm == pytest.approx(np.sqrt(ref * ref - h @ h), rel=200 * EPS["fp64"])

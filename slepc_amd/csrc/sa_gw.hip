@@ -7,9 +7,8 @@
 // w + 8, ...: a chunk is up to NC loads per lane, those of the next chunk in
 // flight while the current one is used.  The update v - V h needs one sum over
 // the waves per chunk (LDS, one barrier that leaves the loads in flight); the
-// dot products accumulate in FP64 registers, FP32 products too one by one (as
-// many instructions as FP32 pairs that are then converted: the same time), and
-// meet in one wave reduction at the end.
+// dot products accumulate in FP64 registers and meet in one wave reduction at
+// the end.
 //
 // HBM bounds it: the basis is read three times per two-pass step, and a slot
 // reads 6.2 TB/s at 57 columns of 2.1M FP64 rows (949 MB in 152 us).  The
@@ -59,6 +58,11 @@ __device__ __forceinline__ void gw_rows(const GsArgs<T> &a, int64_t first, int64
                                         T (*red)[GW_W][64 * VL], double (&acc)[NC], double &self) {
   typedef typename GwVec<T, VL>::type VT;
   constexpr int CR = 64 * VL;
+  // FP32 products against up to 16 columns are added in FP64 one by one: pairs of
+  // a lane's two rows leave 5.3e-11 in the norm of 354,000 rows where the shorter
+  // sums of a 64-row tile left 3.5e-11.  Beyond, those sums had 5 rows and more,
+  // and pairs save 1.5% of a sweep (27-point, 1.3M rows, columns 49-96).
+  constexpr bool ONE = sizeof(T) == 4 && NC <= 2;
   const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = a.c;
   const int64_t nch = (a.n + CR - 1) / CR;
   T *vc = a.V + (int64_t)c * a.ld;
@@ -111,13 +115,23 @@ __device__ __forceinline__ void gw_rows(const GsArgs<T> &a, int64_t first, int64
       }
     }
     if constexpr (DOTS) {
+      T s = (T)0;
 #pragma unroll
-      for (int e = 0; e < VL; e++) self += (double)v[e] * (double)v[e];
+      for (int e = 0; e < VL; e++) {
+        if constexpr (ONE) self += (double)v[e] * (double)v[e];
+        else s += v[e] * v[e];
+      }
+      if constexpr (!ONE) self += (double)s;
 #pragma unroll
       for (int i = 0; i < NC; i++)
         if (i * GW_W + w < c) {
+          T d = (T)0;
 #pragma unroll
-          for (int e = 0; e < VL; e++) acc[i] += (double)x[i][e] * (double)v[e];
+          for (int e = 0; e < VL; e++) {
+            if constexpr (ONE) acc[i] += (double)x[i][e] * (double)v[e];
+            else d += x[i][e] * v[e];
+          }
+          if constexpr (!ONE) acc[i] += (double)d;
         }
     }
   }

@@ -159,10 +159,9 @@ def test_sweep_gives_up_and_starts_over(tmp_path):
     assert float(a["nrm"]) == pytest.approx(float(b["nrm"]), rel=1e-14)
 
 
-# up to 32 columns of the resident sweep, one row and 22 rows per lane; the
-# streaming slots at any width
-@pytest.mark.parametrize("n,j", [(65, 7), (354000, 1), (354000, 10), (354000, 31), (400001, 2), (400001, 60),
-                                 (370001, 110)])
+# up to 32 columns of the resident sweep, one row and 22 rows per lane, and up to
+# 16 of the streaming slots
+@pytest.mark.parametrize("n,j", [(65, 7), (354000, 1), (354000, 10), (354000, 31), (400001, 2), (400001, 16)])
 def test_fp32_products_are_added_in_fp64(sa, n, j):
     """Orthonormalising an FP32 column: coefficients and norm equal those of the
     stored values in FP64.  A product of two FP32 numbers is exact in FP64 and

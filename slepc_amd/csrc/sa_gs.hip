@@ -27,7 +27,8 @@ __global__ void gs_reset_kernel(GsState *st) {
 
 // The three slots of column c and the reductions between them.  The SpMV is a
 // kernel of its own ahead of slot 1: fused into a slot it gathers row by row
-// with every workgroup of the slot waiting for it.
+// with every workgroup of the slot waiting for it.  After a breakdown neither
+// it nor the slots write a column.
 template <typename T>
 static int gs_launch(BV &V, const Mat *A, int c, double eta, hipStream_t s) {
   GsArgs<T> a{};
@@ -38,7 +39,7 @@ static int gs_launch(BV &V, const Mat *A, int c, double eta, hipStream_t s) {
   const bool nt = (int64_t)V.ld * V.m * (int64_t)sizeof(T) > GS_NT_BYTES;
   double *pa = V.ws.part, *pb = V.ws.part + (size_t)V.ws.maxG * (GS_MAXC + 1);
   double *da = V.ws.dots, *db = V.ws.dots + (GS_MAXC + 1);
-  if (A) SA_TRY(launch_spmv(*A, a.V + (size_t)(c - 1) * a.ld, a.V + (size_t)c * a.ld, s));
+  if (A) SA_TRY(launch_spmv(*A, a.V + (size_t)(c - 1) * a.ld, a.V + (size_t)c * a.ld, s, &V.st[2].stop));
   for (int slot = 1; slot <= 3; slot++) {
     a.slot = slot;
     a.part_out = slot == 1 ? pa : pb;

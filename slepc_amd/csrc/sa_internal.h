@@ -139,7 +139,8 @@ constexpr int64_t SPMV_MIN_BLOCKS = 1024;
 int spmv_pick_rows(const int32_t *rp, int64_t n);
 
 // ---- kernel launchers (sa_kernels.hip) -------------------------------------
-int launch_spmv(const Mat &A, const void *x, void *y, hipStream_t s);
+// y = A x; with stop (a device flag) y stays as it is when the flag is set.
+int launch_spmv(const Mat &A, const void *x, void *y, hipStream_t s, const int *stop = nullptr);
 // MatNorm(A, NORM_INFINITY): the largest absolute row sum, computed on the device.
 int mat_norm_inf(const Mat &A, double *out);
 // One Arnoldi/orthonormalisation step for column c of V; spmv_from >= 0 first

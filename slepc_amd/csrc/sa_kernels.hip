@@ -24,23 +24,27 @@ __global__ __launch_bounds__(RBLK) void colsum_kernel(const double *part, int G,
 
 // ---------------------------------------------------------------------------
 // Vector-CSR SpMV: L lanes per row, shuffle reduction (matrices whose row
-// blocks are too dense for the stream kernel below).
+// blocks are too dense for the stream kernel below).  GUARD (in both kernels):
+// y stays as it is once *stop is set, for the steps that a sweep has enqueued
+// beyond a breakdown; the flag is loaded beside the row pointers.
 // ---------------------------------------------------------------------------
-template <typename T, int L>
+template <typename T, int L, bool GUARD>
 __global__ __launch_bounds__(BLK) void spmv_kernel(int n, const int32_t *__restrict__ rp,
                                                    const int32_t *__restrict__ ci,
                                                    const T *__restrict__ val,
-                                                   const T *__restrict__ x, T *__restrict__ y) {
+                                                   const T *__restrict__ x, T *__restrict__ y,
+                                                   const int *__restrict__ stop) {
   const int lg = threadIdx.x % L;
   const int64_t row = ((int64_t)blockIdx.x * BLK + threadIdx.x) / L;
+  const int stopped = GUARD ? *stop : 0;
   T s = (T)0;
   if (row < n) {
-    const int32_t pe = rp[row + 1];
+    const int32_t pe = stopped ? 0 : rp[row + 1];
     for (int32_t p = rp[row] + lg; p < pe; p += L) s += val[p] * x[ci[p]];
   }
 #pragma unroll
   for (int off = L / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, L);
-  if (lg == 0 && row < n) y[row] = s;
+  if (lg == 0 && row < n && !stopped) y[row] = s;
 }
 
 // Stream CSR SpMV for operators larger than the caches: RB rows per
@@ -83,11 +87,11 @@ __device__ __forceinline__ T spmv_row_part(VP vs, CP cs, int b, int e, const T *
   return s;
 }
 
-template <typename T, int RB>
+template <typename T, int RB, bool GUARD>
 __global__ __launch_bounds__(BLK) void spmv_stream_kernel(int n, const int32_t *__restrict__ rp,
                                                           const int32_t *__restrict__ ci,
                                                           const T *__restrict__ val, const T *__restrict__ x,
-                                                          T *__restrict__ y) {
+                                                          T *__restrict__ y, const int *__restrict__ stop) {
   constexpr int TPR = BLK / RB;
   static_assert(RB <= BLK && BLK % RB == 0, "rows per block must divide the workgroup");
   constexpr int NZB = BLK * SPMV_PT;
@@ -99,10 +103,12 @@ __global__ __launch_bounds__(BLK) void spmv_stream_kernel(int n, const int32_t *
   const int t = threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.x * RB;
   const int rows = (int)min((int64_t)RB, (int64_t)n - r0);
+  const int stopped = GUARD ? *stop : 0;
   for (int i = t; i <= rows; i += BLK) srp[i] = rp[r0 + i];
   __syncthreads();
+  if (stopped) return;                   // uniform across the workgroup, as what follows
   const int32_t p0 = srp[0], nz = srp[rows] - p0;
-  const bool staged = nz <= NZB;         // uniform across the workgroup
+  const bool staged = nz <= NZB;
   if (staged) {
     T v[SPMV_PT];
     int32_t c[SPMV_PT];
@@ -148,27 +154,27 @@ __global__ __launch_bounds__(BLK) void spmv_stream_kernel(int n, const int32_t *
   }
 }
 
-template <typename T>
-static int spmv_t(const Mat &A, const T *x, T *y, hipStream_t s) {
-  if (A.spmv_rb > 0) {
-    const int grid = (int)(((int64_t)A.n + A.spmv_rb - 1) / A.spmv_rb);
-    const T *val = (const T *)A.val;
-    switch (A.spmv_rb) {
-      case 256: hipLaunchKernelGGL((spmv_stream_kernel<T, 256>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y); break;
-      case 128: hipLaunchKernelGGL((spmv_stream_kernel<T, 128>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y); break;
-      case 64: hipLaunchKernelGGL((spmv_stream_kernel<T, 64>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y); break;
-      default: hipLaunchKernelGGL((spmv_stream_kernel<T, 32>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y); break;
-    }
-    SA_HIP(hipGetLastError());
-    return 0;
-  }
+template <typename T, bool GUARD>
+static int spmv_t(const Mat &A, const T *x, T *y, const int *stop, hipStream_t s) {
+  const T *val = (const T *)A.val;
+  const bool stream = A.spmv_rb > 0;
   const int64_t threads = (int64_t)A.n * A.lanes;
-  const int grid = (int)((threads + BLK - 1) / BLK);
-  switch (A.lanes) {
-    case 4: hipLaunchKernelGGL((spmv_kernel<T, 4>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, (const T *)A.val, x, y); break;
-    case 8: hipLaunchKernelGGL((spmv_kernel<T, 8>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, (const T *)A.val, x, y); break;
-    case 16: hipLaunchKernelGGL((spmv_kernel<T, 16>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, (const T *)A.val, x, y); break;
-    default: hipLaunchKernelGGL((spmv_kernel<T, 32>), dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, (const T *)A.val, x, y); break;
+  const int grid = (int)(stream ? ((int64_t)A.n + A.spmv_rb - 1) / A.spmv_rb : (threads + BLK - 1) / BLK);
+  auto go = [&](auto *kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y, stop); };
+  if (stream) {
+    switch (A.spmv_rb) {
+      case 256: go(spmv_stream_kernel<T, 256, GUARD>); break;
+      case 128: go(spmv_stream_kernel<T, 128, GUARD>); break;
+      case 64: go(spmv_stream_kernel<T, 64, GUARD>); break;
+      default: go(spmv_stream_kernel<T, 32, GUARD>); break;
+    }
+  } else {
+    switch (A.lanes) {
+      case 4: go(spmv_kernel<T, 4, GUARD>); break;
+      case 8: go(spmv_kernel<T, 8, GUARD>); break;
+      case 16: go(spmv_kernel<T, 16, GUARD>); break;
+      default: go(spmv_kernel<T, 32, GUARD>); break;
+    }
   }
   SA_HIP(hipGetLastError());
   return 0;
@@ -216,10 +222,14 @@ int mat_norm_inf(const Mat &A, double *out) {
   return 0;
 }
 
-int launch_spmv(const Mat &A, const void *x, void *y, hipStream_t s) {
+template <typename T>
+static int spmv_any(const Mat &A, const void *x, void *y, hipStream_t s, const int *stop) {
+  return stop ? spmv_t<T, true>(A, (const T *)x, (T *)y, stop, s) : spmv_t<T, false>(A, (const T *)x, (T *)y, stop, s);
+}
+
+int launch_spmv(const Mat &A, const void *x, void *y, hipStream_t s, const int *stop) {
   if (A.n == 0) return 0;
-  if (A.prec == SA_FP64) return spmv_t<double>(A, (const double *)x, (double *)y, s);
-  return spmv_t<float>(A, (const float *)x, (float *)y, s);
+  return A.prec == SA_FP64 ? spmv_any<double>(A, x, y, s, stop) : spmv_any<float>(A, x, y, s, stop);
 }
 
 // ---------------------------------------------------------------------------

@@ -181,3 +181,31 @@ def test_fp32_products_are_added_in_fp64(sa, n, j):
     assert not lindep
     assert np.abs(H[:j] - h).max() <= 80 * EPS["fp64"] * ref
     assert nrm == pytest.approx(np.sqrt(ref * ref - h @ h), rel=200 * EPS["fp64"])
+
+
+@pytest.mark.parametrize("prec", ["fp64", "fp32"])
+@pytest.mark.parametrize("n,stream", [(3001, False), (400001, False), (400001, True)])
+def test_columns_beyond_a_breakdown_stay(sa, n, stream, prec):
+    """A^2 = 0 on the start vector: the sweep breaks down at column 2 of 7 and
+    leaves the columns after it alone, in the resident kernel and slot by slot
+    with both SpMV layouts."""
+    P = sa.FP64 if prec == "fp64" else sa.FP32
+    # rows 2i take row 2i + 1: with a start vector on the odd rows, A v is on the even ones and A A v = 0
+    r = np.arange(0, n - 1, 2)
+    rp = np.zeros(n + 1, np.int32)
+    rp[1:] = np.cumsum(np.isin(np.arange(n), r))
+    prev = sa.set_spmv_stream_bytes(0) if stream else None
+    M = sa.Mat(sa.CSR(n, rp, (r + 1).astype(np.int32), np.ones(len(r))), P)
+    if stream:
+        sa.set_spmv_stream_bytes(prev)
+    V = sa.BV(n, 8, P)
+    x = np.zeros(n)
+    x[1::2] = 1.0
+    V.set_column(0, x)
+    V.orthonormalize_column(0)
+    for j in range(3, 8):
+        V.set_column(j, np.full(n, 7.0 + j))
+    m, beta, breakdown = V.mat_arnoldi(M, 0, 7)
+    assert (m, beta, breakdown) == (2, 0.0, True)
+    for j in range(3, 8):
+        assert np.all(V.get_column(j) == 7.0 + j)

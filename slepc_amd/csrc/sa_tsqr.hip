@@ -87,6 +87,16 @@ __device__ __forceinline__ void ts_exchange() {
   asm volatile("" ::: "memory");
 }
 
+// Orders a wave's LDS stores before the loads of its other lanes that follow,
+// and its loads before stores that follow.  The hardware keeps a wave's LDS
+// operations in order; without this the compiler need not, as no lane reads
+// what it wrote itself.
+__device__ __forceinline__ void ts_wave_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // The wave's sums of u x[.][c] over its rows for the columns c < KS: lane l
 // returns the one of column l / (64 / SP), SP = ts_pow2(KS).  The first step of
 // the reduce-scatter takes the products as they are formed.
@@ -372,6 +382,7 @@ __global__ __launch_bounds__(64 * W) void tsqr_form_kernel(const T *Y, int64_t l
   for (int rb = 0; rb < RB; rb++) {
 #pragma unroll
     for (int u = 0; u < NU; u++) tr[(4 * u + g) * 17 + c16] = y[rb][u];
+    ts_wave_order();
 #pragma unroll
     for (int h = 0; h < 4; h++) {
       T a[NB];
@@ -383,6 +394,7 @@ __global__ __launch_bounds__(64 * W) void tsqr_form_kernel(const T *Y, int64_t l
 #pragma unroll
         for (int p = q; p < NB; p++, at++) acc[at] = mfma16x16x4(a[q], a[p], acc[at]);
     }
+    ts_wave_order();                            // the next 16 rows overwrite these
   }
   // waves in pairs, the same order every time
 #pragma unroll

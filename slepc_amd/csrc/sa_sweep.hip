@@ -43,16 +43,16 @@
 //
 // All workgroups must be on the GPU together.  The grid has at most one
 // workgroup per CU, and the process admits only sweeps whose workgroups fit
-// the CUs together (ps_admit); kernels of other streams only delay them.  If
+// the CUs together (PsAdmit); kernels of other streams only delay them.  If
 // others hold the CUs all the same (another process), every wait ends after a
 // bounded number of polls, the kernel exits and reports it, and the host runs
 // the sweep slot by slot instead.
 #include <algorithm>
-#include <condition_variable>
 #include <cstdlib>
 #include <mutex>
 #include <vector>
 
+#include "sa_budget.h"
 #include "sa_gs_device.h"
 
 namespace sa {
@@ -595,27 +595,20 @@ __global__ __launch_bounds__(PS_T) void ps_batch_kernel(PsArgs<T> a, const PsPro
 
 // ---- admission: the sweeps in flight together must fit the CUs --------------
 // Workgroups go to the 8 XCDs in turn, so a sweep of G workgroups takes
-// ceil(G / 8) CUs of each; the budget is one XCD's CUs.
-struct PsBudget {
-  std::mutex mu;
-  std::condition_variable cv;
-  int used = 0;
-};
-PsBudget g_budget;
+// ceil(G / 8) CUs of each; the budget is one XCD's CUs, and no sweep takes more
+// workgroups than ps_most().
+int ps_most() { return std::min(num_cus() / N_XCD * N_XCD, 64 * PS_D); }
 
 struct PsAdmit {
-  int units;
-  explicit PsAdmit(int u) : units(u) {
-    std::unique_lock<std::mutex> lk(g_budget.mu);
-    g_budget.cv.wait(lk, [&] { return g_budget.used + units <= num_cus() / N_XCD; });
-    g_budget.used += units;
+  static Budget &budget() {
+    static Budget b(num_cus() / N_XCD);
+    return b;
   }
+  const int units;
+  const bool in;
+  explicit PsAdmit(int G) : units((G + N_XCD - 1) / N_XCD), in(budget().take(units)) {}
   ~PsAdmit() {
-    {
-      std::lock_guard<std::mutex> lk(g_budget.mu);
-      g_budget.used -= units;
-    }
-    g_budget.cv.notify_all();
+    if (in) budget().give(units);
   }
 };
 
@@ -660,9 +653,9 @@ int ps_go(BV &V, const Mat *A, PsArgs<T> &a, hipStream_t s) {
   SA_TRY((ps_room<T, Q>(kern, once, err, &room)));
   if (A) shm = ps_lds<T, Q>(a, room, (double)A->nnz / (double)std::max(1, A->n), V.n);
   a.G = (int)((V.n + R - 1) / R);
-  const int units = (a.G + N_XCD - 1) / N_XCD;
-  PsAdmit admit(units);
   a.host->ok = a.host->fail = 0;
+  PsAdmit admit(a.G);
+  if (!admit.in) return 0;
   hipLaunchKernelGGL(kern, dim3(a.G), dim3(PS_T), shm, s, a);
   SA_HIP(hipGetLastError());
   SA_HIP(hipStreamSynchronize(s));
@@ -695,7 +688,7 @@ int ps_rows(BV &V, const Mat *A, PsArgs<T> &a, int q, hipStream_t s) {
 template <typename T>
 int ps_pick(int64_t n, int S, int share) {
   constexpr int M = sizeof(T) == 8 ? 88 : 176;
-  const int most = std::min(num_cus(), 64 * PS_D);
+  const int most = ps_most();
   for (int want : {share >= 2 ? std::max(64, most / 2) : most, most})
     for (int q : {1, 2, 4, 6, 8, 11, 16, 22}) {
       const int64_t G = (n + 64 * q - 1) / (64 * q);
@@ -749,7 +742,7 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
   }
   SA_TRY(rc);
   *done = a.host->ok && !a.host->fail;
-  if (!*done && !A)   // the vector as it was, for the slots
+  if (a.host->fail && !A)   // the vector as it was, for the slots
     SA_HIP(hipMemcpyAsync(a.V + (size_t)c0 * a.ld, a.backup, sizeof(T) * V.n, hipMemcpyDeviceToDevice, s));
   return 0;
 }
@@ -763,7 +756,11 @@ int psb_go(const PsBatch &w, PsArgs<T> &a, int blocks, double nz_per_row, hipStr
   size_t room;
   SA_TRY((ps_room<T, Q>(kern, once, err, &room)));
   const size_t shm = ps_lds<T, Q>(a, room, nz_per_row, a.xn);
-  PsAdmit admit((blocks + N_XCD - 1) / N_XCD);
+  PsAdmit admit(blocks);
+  if (!admit.in) {
+    w.fail->fail = 1;
+    return 0;
+  }
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(PS_T), shm, s, a, (const PsProb *)w.probs, (const int *)w.of_block);
   SA_HIP(hipGetLastError());
   SA_HIP(hipStreamSynchronize(s));
@@ -783,7 +780,7 @@ int psb_rows(const PsBatch &w, PsArgs<T> &a, int q, int blocks, double nz, hipSt
 template <typename T>
 int psb_run(PsBatch &w, PsArgs<T> &a, std::vector<PsProb> &pr, double nz_per_row, hipStream_t s, bool *done) {
   constexpr int M = sizeof(T) == 8 ? 88 : 176;
-  const int most = std::min(num_cus(), 64 * PS_D);
+  const int most = ps_most();
   int c1 = 0, len = 0;
   int64_t nmax = 0;
   for (const PsProb &p : pr) {

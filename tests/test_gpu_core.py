@@ -453,10 +453,11 @@ def test_concurrent_solves_match_sequential(sa):
 
 
 def test_concurrency_hint_partition(sa, orc):
-    """sa_set_concurrent_solves(4): bases created afterwards use two 64-row
-    chunks per Gram-Schmidt workgroup.  Concurrent solves under the hint give
-    the oracle's eigenvalues (to 1e-10 relative) with every pair at tol, and
-    the same bits as the hinted solves run one after the other."""
+    """sa_set_concurrent_solves(4): concurrent solves under the hint give the
+    oracle's eigenvalues (to 1e-10 relative) with every pair at tol, and the
+    same bits as the hinted solves run one after the other.  (9,216 rows take
+    36 workgroups with and without the hint; sweeps that it halves, and that
+    wait for one another, are in test_gpu_sweep.py.)"""
     import concurrent.futures as cf
     g = 96
     hs = [sa.fv2d(g, g, sa.fv_theta(5, s)) for s in range(4)]

@@ -209,3 +209,32 @@ def test_columns_beyond_a_breakdown_stay(sa, n, stream, prec):
     assert (m, beta, breakdown) == (2, 0.0, True)
     for j in range(3, 8):
         assert np.all(V.get_column(j) == 7.0 + j)
+
+
+def test_concurrent_sweeps_share_the_cus(sa):
+    """Five threads whose sweeps need more than the CUs together (128 workgroups
+    of 65,536 rows with other solves announced, 256 of 180,000): they wait for
+    one another in turn, and each gets the bits that it gets alone."""
+    import concurrent.futures as cf
+
+    def work(n, m, seed):
+        M, V = sa.Mat(_csr(sa, "band", n, seed)), sa.BV(n, m + 1)
+        out = []
+        for k in range(6):
+            V.set_column(0, sa.rand_uniform(seed + k, n))
+            V.orthonormalize_column(0)
+            V.mat_arnoldi(M, 0, m)
+            out.append((V.get_column(m), V.coefficients(1, m + 1)))
+        return out
+
+    jobs = [(65536, 40, 1), (180000, 36, 2), (65536, 40, 3), (180000, 36, 4), (65536, 40, 5)]
+    before = sa.set_concurrent_solves(len(jobs))
+    try:
+        alone = [work(*j) for j in jobs]
+        with cf.ThreadPoolExecutor(len(jobs)) as ex:
+            together = list(ex.map(lambda j: work(*j), jobs))
+    finally:
+        sa.set_concurrent_solves(max(1, before))
+    for a, b in zip(alone, together):
+        for (x, h), (y, g) in zip(a, b):
+            assert np.array_equal(x, y) and np.array_equal(h, g)

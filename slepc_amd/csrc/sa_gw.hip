@@ -2,7 +2,7 @@
 // machine), streaming the basis through registers.
 //
 // A workgroup of 8 waves walks chunks of 128 rows (two per lane; one per lane
-// above 96 FP64 columns) in grid-stride order, so that the workgroups in flight
+// above 96 columns) in grid-stride order, so that the workgroups in flight
 // read one contiguous stretch of every column.  Wave w holds the columns w,
 // w + 8, ...: a chunk is up to NC loads per lane, those of the next chunk in
 // flight while the current one is used.  The update v - V h needs one sum over
@@ -252,7 +252,7 @@ __global__ __launch_bounds__(GW_T) void gw_kernel(GsArgs<T> a) {
 
 template <typename T, int NC>
 void gw_nt(const GsArgs<T> &a, bool nt, hipStream_t s) {
-  constexpr int VL = sizeof(T) == 8 && NC > 12 ? 1 : 2;
+  constexpr int VL = NC > 12 ? 1 : 2;     // two rows of 16 columns spill: FP32 columns 97-126 of 1.3M rows 26.0 ms, one row 12.3
   if (nt) hipLaunchKernelGGL((gw_kernel<T, NC, VL, true>), dim3(a.G), dim3(GW_T), 0, s, a);
   else hipLaunchKernelGGL((gw_kernel<T, NC, VL, false>), dim3(a.G), dim3(GW_T), 0, s, a);
 }

@@ -240,6 +240,10 @@ int sa_bv_resize(sa_bv V, int m, int copy);
 int sa_bv_gs_pass(sa_bv V, int j, double *h_host, double *c_host, double *onorm, double *norm);
 /* Gram-Schmidt passes (CGS1 + DGKS refinements) run on V so far. */
 int sa_bv_get_pass_count(sa_bv V, int64_t *passes);
+/* How the Arnoldi sweeps and orthonormalisations of V have run so far:
+   counts3[0] by the resident kernel, [1] by the slots after a resident kernel
+   gave up waiting, [2] by the slots without one. */
+int sa_bv_get_sweep_counts(sa_bv V, int64_t *counts3);
 
 /* ---- DS: projected dense problem (host FP64, LAPACK) ---------------------------
  * DSSolve + DSSort of a compact DSHEP problem (src/sys/classes/ds/impls/hep/dshep.c:
@@ -533,6 +537,10 @@ int sa_batch_get_stats(sa_batch batch, int64_t *counters6, double *seconds3);
    timings of one sweep (milliseconds, -1 when not timed). */
 int sa_batch_set_sweep(sa_batch batch, int mode);
 int sa_batch_get_sweep(sa_batch batch, int *mode, double *ms_persistent, double *ms_wide);
+/* How the restart sweeps of the batch have run so far, all solves and both
+   precisions, the autotuner's included: counts3[0] resident, [1] lock-step
+   after a resident sweep gave up waiting, [2] lock-step. */
+int sa_batch_get_sweep_counts(sa_batch batch, int64_t *counts3);
 /* The schedule autotuner (mode 0) times, on the first restart round, the
    resident sweep (when ncv < 64) and three lock-step tile schedules:
    the default (non-temporal tile loads for a basis above 256 MiB, SpMV lanes

@@ -373,6 +373,13 @@ class BV:
         check(lib().sa_bv_mat_arnoldi(self.h, A.h, k, C.byref(mm), eta, C.byref(beta), C.byref(bd)))
         return mm.value, beta.value, bool(bd.value)
 
+    def sweep_counts(self):
+        """How sweeps and orthonormalisations have run: by the resident kernel, by
+        the slots after it gave up, by the slots."""
+        c = np.zeros(3, np.int64)
+        check(lib().sa_bv_get_sweep_counts(self.h, c.ctypes.data))
+        return dict(resident=int(c[0]), gave_up=int(c[1]), slots=int(c[2]))
+
     def destroy(self):
         if self.h:
             lib().sa_bv_destroy(self.h)

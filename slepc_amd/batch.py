@@ -23,6 +23,7 @@ def _sig():
     L.sa_batch_set_sweep.argtypes = [vp, C.c_int]
     L.sa_batch_set_true_residual.argtypes = [vp, C.c_int]
     L.sa_batch_get_sweep.argtypes = [vp, C.POINTER(C.c_int), C.POINTER(C.c_double), C.POINTER(C.c_double)]
+    L.sa_batch_get_sweep_counts.argtypes = [vp, vp]
     L.sa_batch_get_schedule.argtypes = [vp, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int), vp]
     L.sa_batch_set_graphs.argtypes = [vp, C.c_int]
     L.sa_batch_get_graph_stats.argtypes = [vp, C.POINTER(C.c_int64), C.POINTER(C.c_int64), C.POINTER(C.c_int)]
@@ -111,6 +112,13 @@ class Batch:
         check(self.L.sa_batch_get_sweep(self.h, C.byref(m), C.byref(a), C.byref(b)))
         names = {v: k for k, v in SWEEP_MODES.items()}
         return dict(mode=names.get(m.value, "none"), ms_persistent=a.value, ms_wide=b.value)
+
+    def sweep_counts(self):
+        """How the restart sweeps have run so far: resident, lock-step after a
+        resident sweep gave up, lock-step."""
+        c = np.zeros(3, np.int64)
+        check(self.L.sa_batch_get_sweep_counts(self.h, c.ctypes.data))
+        return dict(resident=int(c[0]), gave_up=int(c[1]), slots=int(c[2]))
 
     def schedule(self):
         """The last solve's sweep schedule and the autotuner's timings (ms) of the

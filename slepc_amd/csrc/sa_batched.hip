@@ -499,11 +499,13 @@ static int resident_sweep(BatchDev &B, const std::vector<int64_t> &off, const st
 static int run_sweep(BatchDev &B, const Sched &sc, const std::vector<int64_t> &off, const std::vector<int> &nrows,
                      const std::vector<int> &list, const std::vector<int> &k0, const std::vector<int> &nv, int spmv,
                      double eta, hipStream_t s) {
+  const int64_t gave_up = B.ps.tally.gave_up;
   if (sc.kind == 1 && spmv) {
     bool done;
     SA_TRY(resident_sweep(B, off, nrows, list, k0, nv, eta, s, &done));
     if (done) return 0;
   }
+  B.ps.tally.slots += spmv && B.ps.tally.gave_up == gave_up;
   return wide_sweep(B, sc, nrows, list, k0, nv, spmv, eta, s);
 }
 
@@ -562,7 +564,9 @@ static void free_dev(BatchDev &B) {
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   ps_batch_free(B.ps);
+  const SweepTally t = B.ps.tally;
   B = BatchDev();
+  B.ps.tally = t;
 }
 
 static int alloc_dev_impl(sa_batch_s *b, BatchDev &B, int prec, int m);
@@ -1436,6 +1440,15 @@ int sa_batch_get_sweep(sa_batch b, int *mode, double *ms_persistent, double *ms_
   if (mode) *mode = b->sweep_used;
   if (ms_persistent) *ms_persistent = b->ms_persistent;
   if (ms_wide) *ms_wide = b->ms_wide;
+  return 0;
+}
+
+int sa_batch_get_sweep_counts(sa_batch b, int64_t *counts3) {
+  SA_CHECK(b && counts3, "null argument");
+  const SweepTally &x = b->dev64.ps.tally, &y = b->dev32.ps.tally;
+  counts3[0] = x.resident + y.resident;
+  counts3[1] = x.gave_up + y.gave_up;
+  counts3[2] = x.slots + y.slots;
   return 0;
 }
 

@@ -568,6 +568,7 @@ int sa_bv_resize(sa_bv B, int m, int copy) {
   W.l = std::min(V.l, m);
   W.k = std::min(V.k, m);
   W.passes_done = V.passes_done;
+  W.ps.tally = V.ps.tally;
   bv_free(V);
   V = W;
   return 0;
@@ -1413,6 +1414,15 @@ extern "C" {
 int sa_bv_get_pass_count(sa_bv B, int64_t *passes) {
   SA_CHECK(B && passes, "null argument");
   *passes = B->V.passes_done;
+  return 0;
+}
+
+int sa_bv_get_sweep_counts(sa_bv B, int64_t *counts3) {
+  SA_CHECK(B && counts3, "null argument");
+  const SweepTally &t = B->V.ps.tally;
+  counts3[0] = t.resident;
+  counts3[1] = t.gave_up;
+  counts3[2] = t.slots;
   return 0;
 }
 }  // extern "C"

@@ -80,11 +80,18 @@ struct Workspace {           // device scratch for partial sums of one BV
   int maxG = 0;
 };
 
+struct SweepTally {          // how the sweeps of a basis or batch have run
+  int64_t resident = 0;      // by the resident kernel
+  int64_t gave_up = 0;       // by the slots after a resident kernel gave up
+  int64_t slots = 0;         // by the slots
+};
+
 struct PsWork {              // exchange words of the resident sweep (sa_sweep.hip)
   uint64_t *words = nullptr;
   size_t bytes = 0;
   uint32_t tag = 1;          // number of the next exchange
   int share = 1;             // sa_set_concurrent_solves when the basis was created
+  SweepTally tally;
 };
 
 struct PsProb {              // one problem of a batched resident sweep
@@ -101,6 +108,7 @@ struct PsBatch {             // device state of the batched resident sweep
   PsProb *probs = nullptr;
   int *of_block = nullptr;
   GsMirror *fail = nullptr;              // pinned
+  SweepTally tally;                      // of its sweeps with the operator
 };
 
 struct BV {
@@ -151,8 +159,8 @@ int launch_gs_reset(BV &V, hipStream_t s);
 // Columns c0..c1 of V by one resident kernel (sa_sweep.hip): with A each is A
 // times the one before it, orthonormalised; without A, c0 = c1 and column c0
 // itself is.  *done is false when the basis does not fit or the kernel gave
-// up (nothing has changed then); else V.st and V.st_host hold the state.
-// Blocks on the stream.
+// up (the slots can then start at c0); else V.st and V.st_host hold the state.
+// Counted in V.ps.tally.  Blocks on the stream.
 int ps_sweep(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool *done);
 size_t ps_bytes(int64_t n, int prec);   // bytes of its exchange words, 0 when no basis of n rows fits
 // The sweeps of several problems (rows stacked in one basis, block-diagonal

@@ -742,6 +742,8 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
   }
   SA_TRY(rc);
   *done = a.host->ok && !a.host->fail;
+  V.ps.tally.resident += *done;
+  V.ps.tally.gave_up += a.host->fail;
   if (a.host->fail && !A)   // the vector as it was, for the slots
     SA_HIP(hipMemcpyAsync(a.V + (size_t)c0 * a.ld, a.backup, sizeof(T) * V.n, hipMemcpyDeviceToDevice, s));
   return 0;
@@ -826,10 +828,14 @@ int psb_run(PsBatch &w, PsArgs<T> &a, std::vector<PsProb> &pr, double nz_per_row
     SA_HIP(hipMemcpyAsync(w.probs, pr.data() + i0, sizeof(PsProb) * (i1 - i0), hipMemcpyHostToDevice, s));
     SA_HIP(hipMemcpyAsync(w.of_block, of_block.data(), sizeof(int) * blocks, hipMemcpyHostToDevice, s));
     SA_TRY((S == 4 ? psb_rows<T, 4>(w, a, q, blocks, nz_per_row, s) : psb_rows<T, 8>(w, a, q, blocks, nz_per_row, s)));
-    if (w.fail->fail) return 0;
+    if (w.fail->fail) {
+      w.tally.gave_up++;
+      return 0;
+    }
     i0 = i1;
   }
   *done = true;
+  w.tally.resident++;
   return 0;
 }
 
@@ -843,8 +849,11 @@ size_t ps_bytes(int64_t n, int prec) {
 
 int ps_sweep(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool *done) {
   *done = false;
-  if (!V.ps.words || c1 >= GS_MAXC) return 0;
-  return V.prec == SA_FP64 ? ps_run<double>(V, A, c0, c1, eta, s, done) : ps_run<float>(V, A, c0, c1, eta, s, done);
+  const int64_t gave_up = V.ps.tally.gave_up;
+  if (V.ps.words && c1 < GS_MAXC)
+    SA_TRY((V.prec == SA_FP64 ? ps_run<double>(V, A, c0, c1, eta, s, done) : ps_run<float>(V, A, c0, c1, eta, s, done)));
+  V.ps.tally.slots += !*done && V.ps.tally.gave_up == gave_up;
+  return 0;
 }
 
 void ps_batch_free(PsBatch &w) {
@@ -852,7 +861,9 @@ void ps_batch_free(PsBatch &w) {
   if (w.probs) (void)hipFree(w.probs);
   if (w.of_block) (void)hipFree(w.of_block);
   if (w.fail) (void)hipHostFree(w.fail);
+  const SweepTally t = w.tally;
   w = PsBatch();
+  w.tally = t;
 }
 
 bool ps_batch_alloc(PsBatch &w, int64_t nrows, int prec, int P, hipStream_t s) {

@@ -69,10 +69,10 @@ RESIDENT = [
     ([20000] * 9, 24, False), ([20000] * 17 + [33], 24, True)]
 
 
-@pytest.mark.parametrize("rows,ncv,mixed", RESIDENT)
-def test_batched_resident_sweep_edges(sa, rows, ncv, mixed):
+def check_resident(sa, rows, ncv, mixed, ran):
     """The resident sweep and the lock-step one give the same eigenvalues (both
-    have converged to the tolerance) and error estimates below it."""
+    have converged to the tolerance) and error estimates below it.  ran: how
+    the sweeps asked to be resident are to have run."""
     from slepc_amd.batch import Batch
     csrs = [_chain(sa, n, 7 + i % 5) for i, n in enumerate(rows)]
     out = []
@@ -84,7 +84,14 @@ def test_batched_resident_sweep_edges(sa, rows, ncv, mixed):
         assert all(B.converged(p)[2] == 1 for p in range(len(rows)))
         assert np.all(B.errors() <= 1e-10)
         out.append(np.array([[B.eigenpair(p, i, False)[0] for i in range(4)] for p in range(len(rows))]))
+        counts = B.sweep_counts()
+        assert counts[ran if sweep == "persistent" else "slots"] == sum(counts.values()) > 0
     assert np.allclose(out[0], out[1], rtol=1e-10, atol=0)
+
+
+@pytest.mark.parametrize("rows,ncv,mixed", RESIDENT)
+def test_batched_resident_sweep_edges(sa, rows, ncv, mixed):
+    check_resident(sa, rows, ncv, mixed, "resident")
 
 
 GIVE_UP = """
@@ -94,8 +101,8 @@ sys.path.insert(0, %r)
 import slepc_amd as sa
 import test_gpu_batched as t
 sa.init(0)
-t.test_batched_resident_sweep_edges(sa, [2000, 300, 5000], 24, False)
-t.test_batched_resident_sweep_edges(sa, [2000, 300, 5000], 24, True)
+t.check_resident(sa, [2000, 300, 5000], 24, False, "gave_up")
+t.check_resident(sa, [2000, 300, 5000], 24, True, "gave_up")
 """
 
 

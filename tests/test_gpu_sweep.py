@@ -42,7 +42,9 @@ def _matvec(A, X):
     return p[A.rowptr[1:]] - p[A.rowptr[:-1]]
 
 
-def check_relation(sa, n, m, kind, prec):
+def check_relation(sa, n, m, kind, prec, ran="resident"):
+    """ran: how the orthonormalisation of the start vector and the two sweeps are
+    to have run, as BV.sweep_counts names it (or its whole answer)."""
     P = sa.FP64 if prec == "fp64" else sa.FP32
     A = _csr(sa, kind, n)
     if prec == "fp32":
@@ -61,6 +63,7 @@ def check_relation(sa, n, m, kind, prec):
         rel = _matvec(A, X[:, :m]) - X @ np.triu(H, -1)
         assert np.linalg.norm(rel, axis=0).max() <= 40 * (m + 40) * eps
         assert np.abs(X.T @ X - np.eye(m + 1)).max() <= 100 * (m + 1) * eps
+    assert V.sweep_counts() == (ran if isinstance(ran, dict) else dict(dict(resident=0, gave_up=0, slots=0), **{ran: 3}))
 
 
 # rows: one and two chunks, the last row block with one row, exactly 64 blocks
@@ -101,7 +104,8 @@ M = sa.Mat(A)
 V.mat_arnoldi(M, 0, 32)
 V.set_column(33, sa.rand_uniform(6, A.n))
 nrm, lindep = V.orthonormalize_column(33)
-np.savez(sys.argv[1], V=V.get_matrix(34), H=V.coefficients(0, 34), nrm=nrm)
+np.savez(sys.argv[1], V=V.get_matrix(34), H=V.coefficients(0, 34), nrm=nrm,
+         counts=[V.sweep_counts()[k] for k in ("resident", "gave_up", "slots")])
 """
 
 
@@ -112,17 +116,11 @@ sys.path.insert(0, %r)
 import slepc_amd as sa
 import test_gpu_sweep as t
 sa.init(0)
-# a single row, one chunk of 128 rows and its neighbours, more chunks than
-# workgroups; basis widths on both sides of every kernel's column limit
-for n, m, prec in ((1, 1, "fp64"), (127, 17, "fp64"), (128, 33, "fp32"), (129, 49, "fp64"), (3001, 66, "fp64"),
+# one chunk of 128 rows and its neighbours, more chunks than workgroups; basis
+# widths on both sides of every kernel's column limit
+for n, m, prec in ((127, 17, "fp64"), (128, 33, "fp32"), (129, 49, "fp64"), (3001, 66, "fp64"),
                    (3001, 98, "fp64"), (2999, 126, "fp32"), (65663, 30, "fp64"), (65663, 30, "fp32")):
-    if n == 1:
-        V = sa.BV(1, 2)
-        V.set_column(0, [-3.0])
-        nrm, lindep = V.orthonormalize_column(0)
-        assert nrm == 3.0 and not lindep and V.get_column(0)[0] == -1.0
-        continue
-    t.check_relation(sa, n, min(m, n - 1), "band", prec)
+    t.check_relation(sa, n, min(m, n - 1), "band", prec, "gave_up")
     print(n, m, prec, flush=True)
 """
 
@@ -136,7 +134,17 @@ def test_slots_relation():
 
 def test_slots_relation_large(sa):
     """Beyond the registers' capacity, no override needed."""
-    check_relation(sa, 200001, 64, "band", "fp64")
+    check_relation(sa, 200001, 64, "band", "fp64", dict(resident=1, gave_up=0, slots=2))
+    check_relation(sa, 270001, 20, "band", "fp64", "slots")
+
+
+def test_one_row(sa):
+    """A single row: one workgroup, which waits for nobody."""
+    V = sa.BV(1, 2)
+    V.set_column(0, [-3.0])
+    nrm, lindep = V.orthonormalize_column(0)
+    assert nrm == 3.0 and not lindep and V.get_column(0)[0] == -1.0
+    assert V.sweep_counts() == dict(resident=1, gave_up=0, slots=0)
 
 
 def test_sweep_gives_up_and_starts_over(tmp_path):
@@ -154,6 +162,7 @@ def test_sweep_gives_up_and_starts_over(tmp_path):
         subprocess.run([sys.executable, "-c", CODE % ROOT, f], check=True, env=env, timeout=100)
         out.append(np.load(f))
     a, b = out
+    assert a["counts"].tolist() == [3, 0, 0] and b["counts"].tolist() == [0, 3, 0]
     assert np.abs(a["V"] - b["V"]).max() <= 1e-12
     assert np.abs(a["H"] - b["H"]).max() <= 1e-13
     assert float(a["nrm"]) == pytest.approx(float(b["nrm"]), rel=1e-14)

@@ -1,13 +1,16 @@
-// Units of a resource that host threads share, handed out in the order in
-// which the threads ask, so that a large demand is not passed over by small
-// ones.
+// Sharing the GPU between sweeps: a budget for the threads of this process, and
+// when to try again after others were in the way.
 #pragma once
+#include <algorithm>
 #include <condition_variable>
 #include <cstdint>
 #include <mutex>
 
 namespace sa {
 
+// Units of a resource that host threads share, handed out in the order in
+// which the threads ask, so that a large demand is not passed over by small
+// ones.
 class Budget {
  public:
   explicit Budget(int total) : total_(total) {}
@@ -39,6 +42,25 @@ class Budget {
   uint64_t asked_ = 0, served_ = 0;
   std::mutex mu_;
   std::condition_variable cv_;
+};
+
+// After f failures in a row the next 2^(f-1) - 1 turns, 255 at most, pass without
+// a try: one failure costs nothing more, a lasting cause one try in 256 turns.
+class Backoff {
+ public:
+  bool due() {
+    if (rest_ == 0) return true;
+    rest_--;
+    return false;
+  }
+  void succeeded() { failures_ = 0; }
+  void failed() {
+    failures_ = std::min(failures_ + 1, 9);
+    rest_ = (1 << (failures_ - 1)) - 1;
+  }
+
+ private:
+  int failures_ = 0, rest_ = 0;
 };
 
 }  // namespace sa

@@ -6,6 +6,7 @@
 #include <vector>
 
 #include "../../include/slepc_amd.h"
+#include "sa_budget.h"
 
 namespace sa {
 
@@ -92,6 +93,7 @@ struct PsWork {              // exchange words of the resident sweep (sa_sweep.h
   uint32_t tag = 1;          // number of the next exchange
   int share = 1;             // sa_set_concurrent_solves when the basis was created
   SweepTally tally;
+  Backoff backoff;
 };
 
 struct PsProb {              // one problem of a batched resident sweep
@@ -109,6 +111,7 @@ struct PsBatch {             // device state of the batched resident sweep
   int *of_block = nullptr;
   GsMirror *fail = nullptr;              // pinned
   SweepTally tally;                      // of its sweeps with the operator
+  Backoff backoff;
 };
 
 struct BV {
@@ -159,7 +162,7 @@ int launch_gs_reset(BV &V, hipStream_t s);
 // Columns c0..c1 of V by one resident kernel (sa_sweep.hip): with A each is A
 // times the one before it, orthonormalised; without A, c0 = c1 and column c0
 // itself is.  *done is false when the basis does not fit or the kernel gave
-// up (the slots can then start at c0); else V.st and V.st_host hold the state.
+// up (the slots can then start at c0) or is not due after it did; else V.st and V.st_host hold the state.
 // Counted in V.ps.tally.  Blocks on the stream.
 int ps_sweep(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool *done);
 size_t ps_bytes(int64_t n, int prec);   // bytes of its exchange words, 0 when no basis of n rows fits

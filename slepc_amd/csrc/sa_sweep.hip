@@ -46,7 +46,8 @@
 // the CUs together (PsAdmit); kernels of other streams only delay them.  If
 // others hold the CUs all the same (another process), every wait ends after a
 // bounded number of polls, the kernel exits and reports it, and the host runs
-// the sweep slot by slot instead.
+// the sweep slot by slot instead, and after repeated failures those that follow
+// without a try (Backoff).
 #include <algorithm>
 #include <cstdlib>
 #include <mutex>
@@ -698,7 +699,8 @@ int ps_pick(int64_t n, int S, int share) {
 }
 
 // Polls before a wait gives up: about half a second, or SLEPC_AMD_SWEEP_POLLS
-// (0: at the first poll without success, so that every sweep runs by slots).
+// (0: at the first poll without success, so that sweeps of more than one
+// workgroup run by slots).
 int ps_polls() {
   static const int v = [] {
     const char *e = std::getenv("SLEPC_AMD_SWEEP_POLLS");
@@ -712,7 +714,7 @@ template <typename T>
 int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool *done) {
   const int S = c1 <= 32 ? 4 : (c1 <= 64 ? 8 : (c1 <= 96 ? 12 : 16));
   const int q = ps_pick<T>(V.n, S, V.ps.share);
-  if (!q) return 0;
+  if (!q || !V.ps.backoff.due()) return 0;
   PsArgs<T> a{};
   a.n0 = 0; a.n1 = a.xn = V.n; a.ld = V.ld; a.V = static_cast<T *>(V.data);
   if (A) { a.rp = A->rowptr; a.ci = A->col; a.val = static_cast<const T *>(A->val); }
@@ -742,8 +744,13 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
   }
   SA_TRY(rc);
   *done = a.host->ok && !a.host->fail;
-  V.ps.tally.resident += *done;
-  V.ps.tally.gave_up += a.host->fail;
+  if (*done) {
+    V.ps.tally.resident++;
+    V.ps.backoff.succeeded();
+  } else if (a.host->fail) {
+    V.ps.tally.gave_up++;
+    V.ps.backoff.failed();
+  }
   if (a.host->fail && !A)   // the vector as it was, for the slots
     SA_HIP(hipMemcpyAsync(a.V + (size_t)c0 * a.ld, a.backup, sizeof(T) * V.n, hipMemcpyDeviceToDevice, s));
   return 0;
@@ -803,7 +810,7 @@ int psb_run(PsBatch &w, PsArgs<T> &a, std::vector<PsProb> &pr, double nz_per_row
     for (const PsProb &p : pr) total += (p.n1 - p.n0 + 64 * q - 1) / (64 * q);
     if (total <= most) break;
   }
-  if ((nmax + 64 * q - 1) / (64 * q) > most) return 0;
+  if ((nmax + 64 * q - 1) / (64 * q) > most || !w.backoff.due()) return 0;
   const uint32_t tags = 4u * (uint32_t)len + 2u;
   *w.fail = GsMirror{};
   for (size_t i0 = 0; i0 < pr.size();) {
@@ -830,12 +837,14 @@ int psb_run(PsBatch &w, PsArgs<T> &a, std::vector<PsProb> &pr, double nz_per_row
     SA_TRY((S == 4 ? psb_rows<T, 4>(w, a, q, blocks, nz_per_row, s) : psb_rows<T, 8>(w, a, q, blocks, nz_per_row, s)));
     if (w.fail->fail) {
       w.tally.gave_up++;
+      w.backoff.failed();
       return 0;
     }
     i0 = i1;
   }
   *done = true;
   w.tally.resident++;
+  w.backoff.succeeded();
   return 0;
 }
 

@@ -1,5 +1,5 @@
-"""The budget that admits resident sweeps (csrc/sa_budget.h): host code, built
-and run with the host compiler."""
+"""The budget that admits resident sweeps and their back-off
+(csrc/sa_budget.h): host code, built and run with the host compiler."""
 import os
 import shutil
 import subprocess
@@ -79,9 +79,31 @@ static int bounded() {
   return over || done != 1800 ? 2 : 0;
 }
 
+// the turns on which something that always fails is tried, and recovery
+static int backoff() {
+  sa::Backoff b;
+  int tries = 0, last = 0;
+  for (int turn = 1; turn <= 2000; turn++)
+    if (b.due()) {
+      const int gap = turn - last, want = tries == 0 ? 1 : (tries < 9 ? 1 << (tries - 1) : 256);
+      if (gap != want) return 1;
+      tries++;
+      last = turn;
+      b.failed();
+    }
+  while (!b.due()) {
+  }
+  b.succeeded();
+  for (int i = 0; i < 5; i++)
+    if (!b.due()) return 2;
+  b.failed();                    // the first failure after a success is forgiven
+  return b.due() ? 0 : 3;
+}
+
 int main(int, char **v) {
   if (!std::strcmp(v[1], "too_many")) return too_many();
   if (!std::strcmp(v[1], "in_order")) return in_order();
+  if (!std::strcmp(v[1], "backoff")) return backoff();
   return bounded();
 }
 """
@@ -98,9 +120,9 @@ def program(tmp_path_factory):
     return str(d / "t")
 
 
-@pytest.mark.parametrize("what", ["too_many", "in_order", "bounded"])
+@pytest.mark.parametrize("what", ["too_many", "in_order", "bounded", "backoff"])
 def test_budget(program, what):
     """A demand beyond the total is refused instead of awaited, waiting threads
     are served in the order they came, and the units in use never exceed the
-    total."""
+    total; what fails again and again is tried less and less often."""
     assert subprocess.run([program, what], timeout=20).returncode == 0

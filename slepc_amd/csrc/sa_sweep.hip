@@ -350,6 +350,7 @@ __device__ __forceinline__ void ps_block(const PsArgs<T> &a, int b) {
     }
   }
   GsState st = a.st[2];
+  if (b == 0 && t == 0) a.host->passes_before = st.passes_total;
   st.stop = 0; st.stop_col = 0; st.lindep = 0; st.beta = 0.0;
   double hreg = 0.0;                         // coefficient t of the current column (workgroup 0)
   __syncthreads();
@@ -750,6 +751,10 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
   } else if (a.host->fail) {
     V.ps.tally.gave_up++;
     V.ps.backoff.failed();
+    if (a.host->ok) {   // the lead finished, another did not: the slots count these passes again
+      a.host->st.passes_total = a.host->passes_before;
+      SA_HIP(hipMemcpyAsync(V.st + 2, &a.host->st, sizeof(GsState), hipMemcpyHostToDevice, s));
+    }
   }
   if (a.host->fail && !A)   // the vector as it was, for the slots
     SA_HIP(hipMemcpyAsync(a.V + (size_t)c0 * a.ld, a.backup, sizeof(T) * V.n, hipMemcpyDeviceToDevice, s));

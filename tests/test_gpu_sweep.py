@@ -154,6 +154,38 @@ def test_one_row(sa):
     assert V.sweep_counts() == dict(resident=1, gave_up=0, slots=0)
 
 
+PASSES = """
+import ctypes as C, sys
+sys.path.insert(0, %r)
+import slepc_amd as sa
+sa.init(0)
+count = sa.lib().sa_bv_get_pass_count
+count.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
+A = sa.lap2d(70, 61)
+M, p = sa.Mat(A), C.c_int64()
+tally = dict(resident=0, gave_up=0, slots=0)
+for i in range(150):
+    V = sa.BV(A.n, 4)
+    V.set_column(0, sa.rand_uniform(5, A.n))
+    V.scale_column(0, 1.0 / V.norm_column(0))
+    for r in range(1, 5):
+        V.mat_arnoldi(M, 0, 3)
+        sa.check(count(V.h, C.byref(p)))
+        assert p.value == 6 * r, (i, r, p.value, V.sweep_counts())
+    for k, v in V.sweep_counts().items():
+        tally[k] += v
+print(tally)
+"""
+
+
+@pytest.mark.parametrize("polls", ["0", "12", "16"])
+def test_passes_of_a_sweep_that_gave_up_count_once(polls):
+    """Three columns of two passes each, whether the resident kernel finished,
+    gave up (also when its lead workgroup alone finished) or was not tried."""
+    env = dict(os.environ, SLEPC_AMD_SWEEP_POLLS=polls)
+    subprocess.run([sys.executable, "-c", PASSES % ROOT], check=True, env=env, timeout=100)
+
+
 def test_sweep_gives_up_and_starts_over(tmp_path):
     """With no polls allowed, every wait that is not met at once gives up: the
     kernel ends, and the host's slot-by-slot sweep returns the same basis (the

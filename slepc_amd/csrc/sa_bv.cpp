@@ -40,6 +40,7 @@ static int bv_alloc_impl(BV &V, int64_t n, int m, int prec) {
   SA_HIP(hipMalloc(&V.st, sizeof(GsState) * GS_NSTATE));
   SA_HIP(hipMemsetAsync(V.st, 0, sizeof(GsState) * GS_NSTATE, stream()));
   SA_HIP(hipHostMalloc((void **)&V.st_host, sizeof(GsMirror)));
+  std::memset(V.st_host, 0, sizeof(GsMirror));
   // Partition rows into workgroup ranges of whole 64-row chunks.
   const int64_t chunks = std::max<int64_t>(1, (n + 63) / 64);
   // (BVDotVec: at most 1024 workgroups, 4096 for a basis larger than the

@@ -73,7 +73,6 @@ struct GsMirror {   // pinned host memory: the state, and what a resident sweep 
   GsState st;
   int ok;           // its lead workgroup finished
   int fail;         // one of its workgroups gave up waiting
-  int64_t passes_before;   // st.passes_total as the lead workgroup found it
 };
 
 struct Workspace {           // device scratch for partial sums of one BV

@@ -350,7 +350,6 @@ __device__ __forceinline__ void ps_block(const PsArgs<T> &a, int b) {
     }
   }
   GsState st = a.st[2];
-  if (b == 0 && t == 0) a.host->passes_before = st.passes_total;
   st.stop = 0; st.stop_col = 0; st.lindep = 0; st.beta = 0.0;
   double hreg = 0.0;                         // coefficient t of the current column (workgroup 0)
   __syncthreads();
@@ -736,6 +735,7 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
   V.ps.tag += most;
   a.st = V.st; a.host = reinterpret_cast<GsMirror *>(V.st_host); a.dbuf = V.dbuf; a.dm = V.m; a.eta = eta; a.refine = V.refine;
   a.polls = ps_polls();
+  const int64_t passes = a.host->st.passes_total;   // the mirror is the state after every column or sweep
   int rc;
   switch (S) {
     case 4: rc = ps_rows<T, 4>(V, A, a, q, s); break;
@@ -752,7 +752,7 @@ int ps_run(BV &V, const Mat *A, int c0, int c1, double eta, hipStream_t s, bool 
     V.ps.tally.gave_up++;
     V.ps.backoff.failed();
     if (a.host->ok) {   // the lead finished, another did not: the slots count these passes again
-      a.host->st.passes_total = a.host->passes_before;
+      a.host->st.passes_total = passes;
       SA_HIP(hipMemcpyAsync(V.st + 2, &a.host->st, sizeof(GsState), hipMemcpyHostToDevice, s));
     }
   }

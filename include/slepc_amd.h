@@ -531,9 +531,11 @@ int sa_batch_get_stats(sa_batch batch, int64_t *counters6, double *seconds3);
 /* Sweep kernel of the batch: 0 autotune (default; both are timed on the first
    restart round of the first solve phase of each precision and basis width,
    and the faster is kept for later solves of the batch), 1 resident: every
-   problem's basis in the registers of its own workgroups (ncv < 64), 2 lock-step: each Gram-Schmidt
+   problem's basis in the registers of its own workgroups (ncv < 64; a batch
+   with a problem whose basis does not fit them, above 360,448 FP64 rows or
+   180,224 beyond ncv 32, runs lock-step), 2 lock-step: each Gram-Schmidt
    slot of every active problem is one launch over all their 64-row chunks.
-   The getter returns the mode used by the last FP64 phase and the autotuner's
+   The getter returns the mode that the last sweep ran in and the autotuner's
    timings of one sweep (milliseconds, -1 when not timed). */
 int sa_batch_set_sweep(sa_batch batch, int mode);
 int sa_batch_get_sweep(sa_batch batch, int *mode, double *ms_persistent, double *ms_wide);
@@ -546,7 +548,7 @@ int sa_batch_get_sweep_counts(sa_batch batch, int64_t *counts3);
    the default (non-temporal tile loads for a basis above 256 MiB, SpMV lanes
    per row from the mean row length), the other tile-load kind, and twice the
    lanes; it reruns the fastest so the round's results are its own.  The
-   getter returns the last solve's schedule (kind 1 resident,
+   getter returns the last sweep's schedule (kind 1 resident,
    2 lock-step; nt; lanes) and the four timings in milliseconds (-1:
    not timed).  No counterpart in the reference. */
 int sa_batch_get_schedule(sa_batch batch, int *kind, int *nt, int *lanes, double *ms4);

@@ -104,10 +104,12 @@ class Batch:
 
     def set_sweep(self, mode):
         """"auto" (time both sweep kernels on the first restart round), "persistent"
-        (resident: workgroups of its own per problem, ncv < 64) or "wide" (lock-step over row chunks)."""
+        (resident: workgroups of its own per problem, ncv < 64; lock-step where a problem's
+        basis does not fit the registers) or "wide" (lock-step over row chunks)."""
         check(self.L.sa_batch_set_sweep(self.h, SWEEP_MODES[mode]))
 
     def sweep_info(self):
+        """The mode that the last sweep ran in and the autotuner's timings (ms, -1: not timed)."""
         m, a, b = C.c_int(), C.c_double(), C.c_double()
         check(self.L.sa_batch_get_sweep(self.h, C.byref(m), C.byref(a), C.byref(b)))
         names = {v: k for k, v in SWEEP_MODES.items()}

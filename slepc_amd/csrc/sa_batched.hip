@@ -21,6 +21,7 @@
 #include <cstdlib>
 #include <cstring>
 #include <functional>
+#include <limits>
 #include <mutex>
 #include <numeric>
 #include <system_error>
@@ -495,16 +496,18 @@ static int resident_sweep(BatchDev &B, const std::vector<int64_t> &off, const st
 // One sweep of the listed problems with schedule sc (kind 1: resident, 2:
 // lock-step).  Start vectors (no operator) and what the resident sweep does
 // not take go lock-step: it reads columns up to k0 only, so nothing is lost
-// when a resident sweep gave up half-way.
+// when a resident sweep gave up half-way.  *ran: the kind that it ran as.
 static int run_sweep(BatchDev &B, const Sched &sc, const std::vector<int64_t> &off, const std::vector<int> &nrows,
                      const std::vector<int> &list, const std::vector<int> &k0, const std::vector<int> &nv, int spmv,
-                     double eta, hipStream_t s) {
+                     double eta, hipStream_t s, int *ran = nullptr) {
+  if (ran) *ran = 1;
   const int64_t gave_up = B.ps.tally.gave_up;
   if (sc.kind == 1 && spmv) {
     bool done;
     SA_TRY(resident_sweep(B, off, nrows, list, k0, nv, eta, s, &done));
     if (done) return 0;
   }
+  if (ran) *ran = 2;
   B.ps.tally.slots += spmv && B.ps.tally.gave_up == gave_up;
   return wide_sweep(B, sc, nrows, list, k0, nv, spmv, eta, s);
 }
@@ -527,7 +530,7 @@ struct sa_batch_s {
   int P = 0;
   int sweep_req = 0;                    // 0 autotune, 1 persistent, 2 lock-step
   int trueres = 0;                      // EPSSetTrueResidual for every problem
-  int sweep_used = 0;                   // mode of the last solve's FP64 phase
+  int sweep_used = 0;                   // kind that the last restart sweep ran as
   double ms_persistent = -1.0, ms_wide = -1.0;   // autotuner timings of one restart sweep
   int tuned_m[2] = {0, 0};              // basis width the schedule autotuner ran at, per precision (FP64, FP32)
   Sched tuned[2];                       // its choice
@@ -898,6 +901,7 @@ static int batch_ks(sa_batch_s *b, BatchDev &B, int which, int nev, const std::v
     SA_HIP(hipMemcpyAsync(B.k0, k0.data(), sizeof(int) * P, hipMemcpyHostToDevice, s));
     SA_HIP(hipMemcpyAsync(B.nv, nv.data(), sizeof(int) * P, hipMemcpyHostToDevice, s));
     SA_HIP(hipMemcpyAsync(B.stop, stop.data(), sizeof(int) * P, hipMemcpyHostToDevice, s));
+    int ran = 0;
     if (tune) {
       // autotune: the same sweep (it reads only columns <= k0 and rewrites
       // the later ones) with each candidate schedule, timed with events; the
@@ -914,6 +918,7 @@ static int batch_ks(sa_batch_s *b, BatchDev &B, int which, int nev, const std::v
       if (B.lanes < 32) { Sched c = default_sched(B); c.lanes = 2 * B.lanes; cand.push_back(c); cslot.push_back(3); }
       SA_HIP(hipMemcpyAsync(B.passes_save, B.passes, sizeof(int) * P, hipMemcpyDeviceToDevice, s));
       std::vector<float> ms(cand.size(), 0.f);
+      std::vector<int> kind(cand.size(), 2);
       B.graphs_on = false;   // time the kernels, not the first capture of a graph
       hipEvent_t ev[2];
       for (auto &e : ev) SA_HIP(hipEventCreate(&e));
@@ -921,32 +926,43 @@ static int batch_ks(sa_batch_s *b, BatchDev &B, int which, int nev, const std::v
         SA_HIP(hipMemcpyAsync(B.stop, stop.data(), sizeof(int) * P, hipMemcpyHostToDevice, s));
         // the resident sweep's first run allocates its words and loads its
         // code (3.2 ms beside 0.4 ms for the sweep itself)
-        if (cand[c].kind == 1 && !B.ps.words) SA_TRY(run_sweep(B, cand[c], b->off, b->n, act, k0, nv, 1, eta, s));
-        SA_HIP(hipEventRecord(ev[0], s));
-        SA_TRY(run_sweep(B, cand[c], b->off, b->n, act, k0, nv, 1, eta, s));
-        SA_HIP(hipEventRecord(ev[1], s));
-        SA_HIP(hipEventSynchronize(ev[1]));
-        SA_HIP(hipEventElapsedTime(&ms[c], ev[0], ev[1]));
+        bool time_it = true;
+        if (cand[c].kind == 1 && !B.ps.words) {
+          SA_TRY(run_sweep(B, cand[c], b->off, b->n, act, k0, nv, 1, eta, s, &kind[c]));
+          time_it = kind[c] == 1;
+        }
+        if (time_it) {
+          SA_HIP(hipEventRecord(ev[0], s));
+          SA_TRY(run_sweep(B, cand[c], b->off, b->n, act, k0, nv, 1, eta, s, &kind[c]));
+          SA_HIP(hipEventRecord(ev[1], s));
+          SA_HIP(hipEventSynchronize(ev[1]));
+          SA_HIP(hipEventElapsedTime(&ms[c], ev[0], ev[1]));
+        }
+        // a candidate that ran as another one (its basis does not fit, it gave
+        // up) has not been timed
+        if (kind[c] != cand[c].kind) ms[c] = std::numeric_limits<float>::infinity();
       }
       for (auto &e : ev) (void)hipEventDestroy(e);
       const size_t best = std::min_element(ms.begin(), ms.end()) - ms.begin();
       for (int q = 0; q < 4; q++) b->tune_ms[q] = -1.0;
-      for (size_t c = 0; c < cand.size(); c++) b->tune_ms[cslot[c]] = ms[c];
+      for (size_t c = 0; c < cand.size(); c++)
+        if (std::isfinite(ms[c])) b->tune_ms[cslot[c]] = ms[c];
       b->ms_persistent = b->tune_ms[0];
       b->ms_wide = b->tune_ms[1];
       sc = cand[best];
       B.graphs_on = b->graphs;
       SA_HIP(hipMemcpyAsync(B.passes, B.passes_save, sizeof(int) * P, hipMemcpyDeviceToDevice, s));
       SA_HIP(hipMemcpyAsync(B.stop, stop.data(), sizeof(int) * P, hipMemcpyHostToDevice, s));
-      SA_TRY(run_sweep(B, sc, b->off, b->n, act, k0, nv, 1, eta, s));
+      SA_TRY(run_sweep(B, sc, b->off, b->n, act, k0, nv, 1, eta, s, &ran));
       b->tuned_m[pi] = B.m;
       b->tuned[pi] = sc;
       tune = false;
     } else {
-      SA_TRY(run_sweep(B, sc, b->off, b->n, act, k0, nv, 1, eta, s));
+      SA_TRY(run_sweep(B, sc, b->off, b->n, act, k0, nv, 1, eta, s, &ran));
     }
-    b->sweep_used = sc.kind;
+    b->sweep_used = ran;
     b->sched_used = sc;
+    b->sched_used.kind = ran;
     // coefficients of the problems from the first to the last active one
     const int plo = *std::min_element(act.begin(), act.end()), phi = *std::max_element(act.begin(), act.end());
     dbuf.resize((size_t)P * m * m);

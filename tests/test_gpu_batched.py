@@ -80,7 +80,7 @@ def check_resident(sa, rows, ncv, mixed, ran):
         B = Batch(csrs)
         B.set_sweep(sweep)
         B.solve(4, ncv, 1e-10, "LM", mixed=mixed)
-        assert B.sweep_info()["mode"] == sweep
+        assert B.sweep_info()["mode"] == ("persistent" if sweep == "persistent" and ran == "resident" else "wide")
         assert all(B.converged(p)[2] == 1 for p in range(len(rows)))
         assert np.all(B.errors() <= 1e-10)
         out.append(np.array([[B.eigenpair(p, i, False)[0] for i in range(4)] for p in range(len(rows))]))
@@ -95,6 +95,18 @@ def check_resident(sa, rows, ncv, mixed, ran):
 @pytest.mark.parametrize("rows,ncv,mixed", RESIDENT)
 def test_batched_resident_sweep_edges(sa, rows, ncv, mixed):
     check_resident(sa, rows, ncv, mixed, "resident")
+
+
+def test_batched_beyond_the_registers(sa):
+    """A problem of one row more than 256 workgroups hold: "persistent" and the
+    autotuner run lock-step and say so, and the resident sweep is not timed."""
+    check_resident(sa, [256 * 64 * 22 + 1, 100], 12, False, "slots")
+    from slepc_amd.batch import Batch
+    B = Batch([_chain(sa, n, 7) for n in (256 * 64 * 22 + 1, 100)])
+    B.solve(4, 12, 1e-10, "LM")
+    info, sched = B.sweep_info(), B.schedule()
+    assert info["mode"] == sched["kind"] == "wide" and info["ms_persistent"] == -1.0 and info["ms_wide"] > 0.0
+    assert sched["ms"][0] == -1.0 and B.sweep_counts()["resident"] == 0
 
 
 GIVE_UP = """

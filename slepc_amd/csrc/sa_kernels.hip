@@ -406,7 +406,7 @@ __global__ __launch_bounds__(BLK) void multinplace_kernel(int64_t n, int64_t ld,
 constexpr size_t MIP_QS_BYTES = 64 * 1024;
 // Workgroups (each stages Q once): whole rounds of those that are resident
 // together, four per CU with one row per lane, two of the three that fit with 16
-// bytes, or two rounds of three for short products (1.5M rows, K = 64, N = 32 FP64 with 512, 1024, 1536: 252, 287, 250 us).
+// bytes (1.5M rows, K = 64, N = 32 FP64 with 512, 1024, 1536: 252, 287, 250 us).
 constexpr int64_t MIP_GRID = 1024;
 
 template <typename T, int NTL, int VL, bool NT>
@@ -443,7 +443,7 @@ __global__ __launch_bounds__(BLK) void multinplace_q_kernel(int64_t n, int64_t l
         const T *p = src + (size_t)kk * ld;
         if (whole) {
           an[u] = ld_stream<NT>(reinterpret_cast<const VT *>(p));
-        } else {
+        } else if constexpr (VL > 1) {
 #pragma unroll
           for (int e = 0; e < VL; e++)
             if (row + e < n) an[u][e] = p[e];
@@ -492,7 +492,7 @@ __global__ __launch_bounds__(BLK) void multinplace_q_kernel(int64_t n, int64_t l
         for (int e = 0; e < VL; e++) o[e] = acc[e][q][v];
         if (row + VL <= n) {
           *reinterpret_cast<VT *>(dst + (size_t)j * ld) = o;
-        } else {
+        } else if constexpr (VL > 1) {
 #pragma unroll
           for (int e = 0; e < VL; e++)
             if (row + e < n) dst[(size_t)j * ld + e] = o[e];
@@ -504,7 +504,7 @@ __global__ __launch_bounds__(BLK) void multinplace_q_kernel(int64_t n, int64_t l
 template <typename T, int NTL, int VL>
 static void launch_mip_rows(BV &V, int l, int K, int s_, int N, const double *Q_dev, int ldq, hipStream_t s) {
   const int64_t rows = 4 * 16 * VL;                // per workgroup step
-  const int most = VL == 1 ? MIP_GRID : (NTL == 1 ? 3 * MIP_GRID / 2 : MIP_GRID / 2);
+  const int most = VL == 1 ? MIP_GRID : MIP_GRID / 2;
   const int grid = (int)std::min<int64_t>((V.n + rows - 1) / rows, most);
   const size_t shm = (size_t)((K + 3) & ~3) * (NTL * 16 + 1) * sizeof(T);
   if (V.n * (int64_t)K * (int64_t)sizeof(T) > GS_NT_BYTES)
@@ -517,17 +517,28 @@ static void launch_mip_rows(BV &V, int l, int K, int s_, int N, const double *Q_
 
 template <typename T, int NTL>
 static void launch_mip_q(BV &V, int l, int K, int s_, int N, const double *Q_dev, int ldq, hipStream_t s) {
-  constexpr int VL = 16 / (int)sizeof(T);
-  // 16 bytes per lane, or one row per lane for few output columns and on small
-  // blocks, where more waves count (microseconds with 16 bytes and with one row,
-  // FP64: K = 30, N = 15 at 1.5M rows 106.8, 108.3, K = 20, N = 10 at 300,000 32.8, 30.4;
-  // K = 61, N = 34 at 159,556 57.7, 57.5, K = 40, N = 20 at 250,000 45.6, 44.0, K = 61,
-  // N = 33 at 180,000 56.4, 57.4, K = 64, N = 48 at 200,000 66.8, 69.9, K = 80, N = 40 at
-  // 400,000 104.6, 116.6; FP32 four rows per lane: at 100,000 53.2, 50.4)
-  constexpr int64_t M = (int64_t)1 << 20, from = sizeof(T) == 8 ? (NTL > 1 ? 10 * M : 32 * M) : 16 * M;
-  constexpr bool wide = sizeof(T) == 8 || NTL > 1;
-  if (wide && V.n * K >= from) launch_mip_rows<T, NTL, VL>(V, l, K, s_, N, Q_dev, ldq, s);
-  else launch_mip_rows<T, NTL, 1>(V, l, K, s_, N, Q_dev, ldq, s);
+  // 16 bytes per lane, or one row per lane with up to 16 output columns and on
+  // small blocks, where more waves count.  The line lies where it does because a
+  // Q value from LDS serves 2 or 4 products: the more output tiles, the earlier
+  // that pays.  Microseconds with 16 bytes and with one row, FP64:
+  //   up to 16 columns: rows, K -> N 900,000, 40 -> 10 88.6, 80.6; 1.5M, 30 -> 15
+  //     109.9, 105.6; 4M, 24 -> 12 250, 246 (2^21 rows alone favour 16 bytes: 32 ->
+  //     16 153.6, 156.0);
+  //   up to 32, from 10M elements of the basis block: 90,000, 50 -> 25 35.6, 34.5;
+  //     70,000, 64 -> 32 38.5, 35.8; 250,000, 40 -> 20 46.5, 45.6; then 350,000, 32 ->
+  //     32 48.6, 50.6; 250,000, 48 -> 24 49.6, 51.9; 200,000, 64 -> 32 53.0, 55.0;
+  //   more, from 4M: 30,000, 90 -> 70 54.9, 52.1; 30,000, 100 -> 48 48.2, 47.5; then
+  //     50,000, 90 -> 48 55.0, 54.3; 70,000, 64 -> 48 50.7, 50.5; 100,000, 90 -> 48 65.2,
+  //     65.2; 159,556, 61 -> 34 63.4, 64.2; 180,000, 61 -> 33 58.2, 59.8; 120,000, 64 ->
+  //     64 63.0, 72.1; 60,000, 100 -> 80 68.1, 76.1; 400,000, 80 -> 40 111, 129.
+  // FP32, from 16M: 150,000, 100 -> 64 80.7, 76.6; then 300,000, 64 -> 32 49.5, 49.9;
+  // 300,000, 64 -> 48 65.4, 69.5; 600,000, 48 -> 24 55.7, 61.9.
+  if constexpr (NTL > 1) {
+    constexpr int VL = 16 / (int)sizeof(T);
+    constexpr int64_t M = (int64_t)1 << 20, from = sizeof(T) == 8 ? (NTL > 2 ? 4 * M : 10 * M) : 16 * M;
+    if (V.n * K >= from) return launch_mip_rows<T, NTL, VL>(V, l, K, s_, N, Q_dev, ldq, s);
+  }
+  launch_mip_rows<T, NTL, 1>(V, l, K, s_, N, Q_dev, ldq, s);
 }
 
 template <typename T>

@@ -347,9 +347,27 @@ def test_tsqr_tile_edges(sa, n, k, prec):
 @pytest.mark.parametrize("n,K,N", [(15, 5, 3), (65, 33, 17), (65537, 33, 16), (66049, 40, 49), (131201, 20, 7),
                                    (140003, 96, 48)])
 def test_restart_product_row_blocks(sa, n, K, N, prec):
-    """BVMultInPlace at the edges of its row blocks (one row per lane, 16 bytes
-    per lane from 65,536 rows on, ragged last blocks, more blocks than
-    workgroups) against the product in FP64: K rounded products per entry."""
+    """BVMultInPlace at the edges of its row blocks (one row per lane, but 16
+    bytes for the last in FP64; ragged last blocks, more blocks than workgroups)
+    against the product in FP64: K rounded products per entry."""
+    check_restart_product(sa, n, K, N, prec)
+
+
+# either side of the lines from which 16 bytes per lane are taken: FP64 4M
+# elements with more than 32 output columns, 10M with more than 16 (never with
+# fewer), FP32 16M with more than 16; there every remainder of the 2 or 4 rows
+# of a lane, batches of 8 and 4 k-steps (4 beyond 8 tiles of a lane's rows), more
+# row blocks than waves
+@pytest.mark.parametrize("n,K,N,prec", [
+    (65535, 64, 33, "fp64"), (65537, 64, 33, "fp64"), (65539, 64, 64, "fp64"), (44001, 96, 67, "fp64"),
+    (131075, 84, 83, "fp64"), (163839, 64, 32, "fp64"), (163841, 64, 32, "fp64"), (600001, 20, 17, "fp64"),
+    (900001, 40, 10, "fp64"), (262143, 64, 32, "fp32"), (262145, 64, 17, "fp32"), (262146, 64, 32, "fp32"),
+    (174763, 97, 48, "fp32"), (174765, 96, 64, "fp32"), (139815, 120, 96, "fp32")])
+def test_restart_product_either_side_of_the_lines(sa, n, K, N, prec):
+    check_restart_product(sa, n, K, N, prec)
+
+
+def check_restart_product(sa, n, K, N, prec):
     P = sa.FP64 if prec == "fp64" else sa.FP32
     eps = EPS if prec == "fp64" else 6e-8
     rng = np.random.default_rng(n + K)

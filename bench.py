@@ -82,9 +82,14 @@ A64_nnz = [0]
 def sweep_roofline(sa, A64, n, m):
     """One m-step Arnoldi sweep (the resident kernel, or SpMV, Gram-Schmidt
     slots and their one-workgroup reductions only), timed with HIP events on the library
-    stream.  Algorithmic bytes: per step the SpMV (values, indices, row
-    pointers, x, y) and per Gram-Schmidt pass 2(c+1) basis columns (dots read
-    c columns, the update reads c columns and v and writes v)."""
+    stream.  Bytes: slot by slot the algorithmic ones, per step the SpMV (values,
+    indices, row pointers, x, y) and per Gram-Schmidt pass 2(c+1) basis columns
+    (dots read c columns, the update reads c columns and v and writes v; the
+    slots read the basis for a pass's update and the next one's dots together
+    and move about three quarters of that); by the resident kernel, which keeps
+    operator and basis on the chip, those that have to move: the operator and
+    the first column once and each new column once.  Returns GB/s, bytes,
+    milliseconds, passes per step and whether the sweep ran resident."""
     L = sa.lib()
     L.sa_bv_get_pass_count.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
     V = sa.BV(n, m + 1, sa.FP64)
@@ -95,18 +100,23 @@ def sweep_roofline(sa, A64, n, m):
     V.orthonormalize_column(0)
     p0, p1 = C.c_int64(), C.c_int64()
     sa.check(L.sa_bv_get_pass_count(V.h, C.byref(p0)))
+    before = V.sweep_counts()["resident"]
     sa.check(L.sa_timer_start())
     mm, beta, bd = V.mat_arnoldi(A64, 0, m)
     ms = C.c_double()
     sa.check(L.sa_timer_stop(C.byref(ms)))
     sa.check(L.sa_bv_get_pass_count(V.h, C.byref(p1)))
     passes = (p1.value - p0.value) / float(mm)
+    resident = V.sweep_counts()["resident"] > before
     for _ in range(3):                    # device copies of one column: traffic calibration for counter runs
         V.copy_column(0, 1)
-    spmv = A64_nnz[0] * 12.0 + 4.0 * (n + 1) + 16.0 * n
-    bv = sum(passes * (2.0 * c + 2.0) * n * 8.0 for c in range(1, mm + 1))
-    total = mm * spmv + bv
-    return total / (ms.value * 1e-3) / 1e9, total, ms.value, passes
+    operator = A64_nnz[0] * 12.0 + 4.0 * (n + 1)
+    if resident:
+        total = operator + 8.0 * n * (1 + mm)
+    else:
+        bv = sum(passes * (2.0 * c + 2.0) * n * 8.0 for c in range(1, mm + 1))
+        total = mm * (operator + 16.0 * n) + bv
+    return total / (ms.value * 1e-3) / 1e9, total, ms.value, passes, resident
 
 
 def spmv_roofline(sa, Ah, reps=10):
@@ -268,7 +278,7 @@ def run_scale(sa):
     Ch = sa.convdiff3d(128)
     C64 = sa.Mat(Ch, sa.FP64)
     A64_nnz[0] = Ch.nnz
-    gbs2, tb2, ms2, p2 = sweep_roofline(sa, C64, Ch.n, 64)
+    gbs2, tb2, ms2, p2, _ = sweep_roofline(sa, C64, Ch.n, 64)
     # non-normal operator: the true residual exceeds the Ritz estimate, so
     # the convergence test takes explicit residuals (EPSSetTrueResidual);
     # without locking (EPSKrylovSchurSetLocking 0) the converged vectors keep
@@ -297,7 +307,7 @@ def run_scale(sa):
     s3 = {"workload": "27-pt 128^3 + diag U[0,1] seed 1 (n=2,097,152, nnz 55,742,968) HEP, nev 32 largest "
                       "magnitude, ncv 96, tol 1e-10"}
     A64_nnz[0] = Sh.nnz
-    gbs3, tb3, ms3, p3 = sweep_roofline(sa, S64, Sh.n, 96)
+    gbs3, tb3, ms3, p3, _ = sweep_roofline(sa, S64, Sh.n, 96)
     s3.update({"gs_sweep_GBs": round(gbs3, 1), "gs_sweep_frac": round(gbs3 / HBM_PEAK_GBS, 4),
                "gs_sweep_ms": round(ms3, 3), "gs_sweep_passes_per_step": p3, "spmv": spmv_roofline(sa, Sh)})
     vals = {}
@@ -428,9 +438,9 @@ def main():
             Ah = (sa.fv2d(GRID, GRID, sa.fv_theta(THETA_SEED_TEST, 0)) if name == "fv2d_256" else
                   sa.convdiff3d(128) if name == "convdiff_128" else sa.stencil27(128, seed=1))
             A64_nnz[0] = Ah.nnz
-            gbs, tb, ms, passes = sweep_roofline(sa, sa.Mat(Ah), Ah.n, 96 if name == "stencil27_128" else NCV)
+            gbs, tb, ms, passes, resident = sweep_roofline(sa, sa.Mat(Ah), Ah.n, 96 if name == "stencil27_128" else NCV)
             out[name] = {"GBs": round(gbs, 1), "frac": round(gbs / HBM_PEAK_GBS, 4), "ms": round(ms, 3),
-                         "bytes": tb, "passes_per_step": passes}
+                         "bytes": tb, "passes_per_step": passes, "resident": resident}
             if args.spmv:
                 out[name]["spmv"] = spmv_roofline(sa, Ah)
                 if name == "stencil27_128":
@@ -494,14 +504,17 @@ def main():
 
     # ---------------- roofline of the Arnoldi sweep kernels
     A64_nnz[0] = probs[0][1].nnz
-    gbs, tot_bytes, ms, passes = sweep_roofline(sa, probs[0][2], n, NCV)
-    roof = {"bound": "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-            "frac": round(gbs / HBM_PEAK_GBS, 4), "traffic": profiled_traffic("fv2d_256"),
-            "kernel": "ps_sweep_kernel (resident SpMV + CGS + DGKS), one launch = one 64-step sweep",
+    gbs, tot_bytes, ms, passes, resident = sweep_roofline(sa, probs[0][2], n, NCV)
+    roof = {"bound": "latency" if resident else "hbm", "achieved": round(gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+            "frac": round(gbs / HBM_PEAK_GBS, 4), "us_per_step": round(ms * 1e3 / NCV, 2),
+            "traffic": profiled_traffic("fv2d_256"),
+            "kernel": "ps_sweep_kernel (resident SpMV + CGS + DGKS), one launch = one 64-step sweep" if resident else
+                      "SpMV, gw_kernel slots and gs_sum_kernel, six launches per step",
             "note": "64-step Arnoldi sweep on the headline operator (n=65,536, %.2f passes/step): %.1f MB "
-                    "algorithmic in %.3f ms (HIP events); the 34 MB basis stays in registers and the exchanges between "
-                    "workgroups (about 1.3 us each, five per step) bound it; traffic = counter-measured HBM bytes per sweep "
-                    "from profiles/gs_sweep_fv2d_256.txt" % (passes, tot_bytes / 1e6, ms)}
+                    "have to move, in %.3f ms (HIP events).  Resident, the 34 MB basis stays in registers and the "
+                    "exchanges between workgroups (about 1.3 us each, five per step) bound the sweep, not HBM; traffic = "
+                    "counter-measured HBM bytes per sweep from profiles/gs_sweep_fv2d_256.txt (exchange words and "
+                    "fetched halo entries included)" % (passes, tot_bytes / 1e6, ms)}
 
     roof["spmv_fv2d_256"] = spmv_roofline(sa, probs[0][1])
 

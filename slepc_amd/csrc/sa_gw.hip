@@ -16,8 +16,10 @@
 // and nothing in flight across them, and reached 4.9 TB/s.  Sweeps at 128^3:
 // convection-diffusion FP64, columns 33-64, 17.5 -> 14.1 ms; 27-point FP64,
 // columns 49-96, 44.9 -> 34.9 ms; columns 97-124, 42.8 -> 30.0 ms; 27-point FP32,
-// 1.3M rows, columns 49-96, 16.3 -> 11.8 ms.  At 110,000 to 400,000 rows it
-// takes 0.8-0.95 of the time, at 2,500 to 10,000 about the same.
+// 1.3M rows, columns 49-96, 16.3 -> 11.8 ms, 97-126, 15.5 -> 12.4.  Bases of FP64 in
+// the last-level cache gain least: 5-point, columns 33-64, 240,000 rows 2.32 ->
+// 2.08 ms, 300,000 2.71 -> 2.50, 399,000 3.41 -> 3.09; 300,000 rows, columns 1-30
+// 1.56 -> 1.31, 49-96 6.98 -> 5.06.
 #include <algorithm>
 
 #include "sa_gs_device.h"

@@ -37,9 +37,9 @@
 // What bounds it is the latency of the five exchanges of a step, about 1.3 us
 // each (a store to memory and a load that misses the L2): of 10-11 us per step
 // at n = 10,000 and 65,536 they take 7, the decision and the update 2, the dot
-// products 0.7.  Measured against the slots: 64 steps at n = 65,536 790 us
-// (1,850), 16 steps from column 16 at n = 10,000 198 us (360), FP32 32 steps
-// from column 32 at n = 354,000 602 us (2,504).
+// products 0.7.  Measured against the slots of 64-row tiles: 64 steps at n =
+// 65,536 770 us (1,880), 16 steps from column 16 at n = 10,000 200 us (374), FP32
+// 32 steps from column 32 at n = 354,000 628 us (2,479).
 //
 // All workgroups must be on the GPU together.  The grid has at most one
 // workgroup per CU, and the process admits only sweeps whose workgroups fit
@@ -678,7 +678,7 @@ int ps_rows(BV &V, const Mat *A, PsArgs<T> &a, int q, hipStream_t s) {
 
 // 64-row chunks per workgroup for n rows and S column slots, 0 when the basis
 // does not fit.  A thread keeps S * Q values: at most 88 doubles or 176 floats
-// (the largest spill up to 144 B per lane and still take 0.4 of the slots'
+// (the largest spill up to 136 B per lane and still take 0.4 of the slots'
 // time).  Up to 64 workgroups, or 4 chunks each, more rows per workgroup cost
 // nothing (n = 10,000: 198, 200, 198 us with 1, 2, 4 chunks) and leave CUs to
 // the sweeps of other threads; beyond that as few rows as the CUs allow.  When

@@ -322,7 +322,8 @@ struct TsForm {
 // in LDS) and Y X are matrix products on the MFMA units and what is left, k x k
 // per tile, is a triangular solve.  Memory bounds it (the level over V of 2.1M
 // rows and 32 columns FP64 takes 386 us, 226 at the copy rate), then the solve,
-// which only the two tiles a CU holds overlap.  Against applying the
+// which only the two tiles a CU holds overlap (64 columns FP64 spill 104 bytes per
+// lane beside that).  Against applying the
 // reflectors one by one, each a reduction and an update of all columns (the
 // whole factorization, 2.1M rows FP64): 16 columns 523 -> 481 us, 24 950 -> 874,
 // 32 1471 -> 1301, 48 4.9 -> 3.4 ms, 64 7.2 -> 5.0; 8 columns, which the matrix units

@@ -24,29 +24,25 @@ __global__ __launch_bounds__(RBLK) void colsum_kernel(const double *part, int G,
 
 // ---------------------------------------------------------------------------
 // Vector-CSR SpMV: L lanes per row, shuffle reduction (matrices whose row
-// blocks are too dense for the stream kernel below).  GUARD (in both kernels):
-// y stays as it is once *stop is set, for the steps that a sweep has enqueued
-// beyond a breakdown.  The flag is a vector load beside the row pointers that
-// only the stores wait for: as a scalar load that every LDS wait includes it
-// cost 4.5 us of a 57 us product (27-point, FP32, 1.3M rows), so 0.9.
+// blocks are too dense for the stream kernel below).  The _unless kernels leave
+// y as it is once *stop is set, for the steps that a sweep has enqueued beyond a
+// breakdown.
 // ---------------------------------------------------------------------------
-template <bool GUARD>
+// The flag as a vector load beside the row pointers that only the stores wait
+// for: as a scalar load that every LDS wait includes it cost 4.5 us of a 57 us
+// product (27-point, FP32, 1.3M rows), so 0.9.
 __device__ __forceinline__ int spmv_stopped(const int *stop) {
-  if constexpr (!GUARD) return 0;
   int lane0 = 0;
   asm volatile("" : "+v"(lane0));        // an address in vector registers
   return stop[lane0];
 }
 
-template <typename T, int L, bool GUARD>
-__global__ __launch_bounds__(BLK) void spmv_kernel(int n, const int32_t *__restrict__ rp,
-                                                   const int32_t *__restrict__ ci,
-                                                   const T *__restrict__ val,
-                                                   const T *__restrict__ x, T *__restrict__ y,
-                                                   const int *__restrict__ stop) {
+template <typename T, int L>
+__device__ __forceinline__ void spmv_rows(int n, const int32_t *__restrict__ rp, const int32_t *__restrict__ ci,
+                                          const T *__restrict__ val, const T *__restrict__ x, T *__restrict__ y,
+                                          int stopped) {
   const int lg = threadIdx.x % L;
   const int64_t row = ((int64_t)blockIdx.x * BLK + threadIdx.x) / L;
-  const int stopped = spmv_stopped<GUARD>(stop);
   T s = (T)0;
   if (row < n) {
     const int32_t pe = rp[row + 1];
@@ -55,6 +51,22 @@ __global__ __launch_bounds__(BLK) void spmv_kernel(int n, const int32_t *__restr
 #pragma unroll
   for (int off = L / 2; off > 0; off >>= 1) s += __shfl_xor(s, off, L);
   if (lg == 0 && row < n && !stopped) y[row] = s;
+}
+
+template <typename T, int L>
+__global__ __launch_bounds__(BLK) void spmv_kernel(int n, const int32_t *__restrict__ rp,
+                                                   const int32_t *__restrict__ ci,
+                                                   const T *__restrict__ val,
+                                                   const T *__restrict__ x, T *__restrict__ y) {
+  spmv_rows<T, L>(n, rp, ci, val, x, y, 0);
+}
+
+template <typename T, int L>
+__global__ __launch_bounds__(BLK) void spmv_unless_kernel(int n, const int32_t *__restrict__ rp,
+                                                          const int32_t *__restrict__ ci, const T *__restrict__ val,
+                                                          const T *__restrict__ x, T *__restrict__ y,
+                                                          const int *__restrict__ stop) {
+  spmv_rows<T, L>(n, rp, ci, val, x, y, spmv_stopped(stop));
 }
 
 // Stream CSR SpMV for operators larger than the caches: RB rows per
@@ -97,11 +109,10 @@ __device__ __forceinline__ T spmv_row_part(VP vs, CP cs, int b, int e, const T *
   return s;
 }
 
-template <typename T, int RB, bool GUARD>
-__global__ __launch_bounds__(BLK) void spmv_stream_kernel(int n, const int32_t *__restrict__ rp,
-                                                          const int32_t *__restrict__ ci,
-                                                          const T *__restrict__ val, const T *__restrict__ x,
-                                                          T *__restrict__ y, const int *__restrict__ stop) {
+template <typename T, int RB>
+__device__ __forceinline__ void spmv_stream_block(int n, const int32_t *__restrict__ rp,
+                                                  const int32_t *__restrict__ ci, const T *__restrict__ val,
+                                                  const T *__restrict__ x, T *__restrict__ y, int stopped) {
   constexpr int TPR = BLK / RB;
   static_assert(RB <= BLK && BLK % RB == 0, "rows per block must divide the workgroup");
   constexpr int NZB = BLK * SPMV_PT;
@@ -113,7 +124,6 @@ __global__ __launch_bounds__(BLK) void spmv_stream_kernel(int n, const int32_t *
   const int t = threadIdx.x;
   const int64_t r0 = (int64_t)blockIdx.x * RB;
   const int rows = (int)min((int64_t)RB, (int64_t)n - r0);
-  const int stopped = spmv_stopped<GUARD>(stop);
   for (int i = t; i <= rows; i += BLK) srp[i] = rp[r0 + i];
   __syncthreads();
   const int32_t p0 = srp[0], nz = srp[rows] - p0;
@@ -163,26 +173,45 @@ __global__ __launch_bounds__(BLK) void spmv_stream_kernel(int n, const int32_t *
   }
 }
 
-template <typename T, bool GUARD>
+template <typename T, int RB>
+__global__ __launch_bounds__(BLK) void spmv_stream_kernel(int n, const int32_t *__restrict__ rp,
+                                                          const int32_t *__restrict__ ci,
+                                                          const T *__restrict__ val, const T *__restrict__ x,
+                                                          T *__restrict__ y) {
+  spmv_stream_block<T, RB>(n, rp, ci, val, x, y, 0);
+}
+
+template <typename T, int RB>
+__global__ __launch_bounds__(BLK) void spmv_stream_unless_kernel(int n, const int32_t *__restrict__ rp,
+                                                                 const int32_t *__restrict__ ci,
+                                                                 const T *__restrict__ val, const T *__restrict__ x,
+                                                                 T *__restrict__ y, const int *__restrict__ stop) {
+  spmv_stream_block<T, RB>(n, rp, ci, val, x, y, spmv_stopped(stop));
+}
+
+template <typename T>
 static int spmv_t(const Mat &A, const T *x, T *y, const int *stop, hipStream_t s) {
   const T *val = (const T *)A.val;
   const bool stream = A.spmv_rb > 0;
   const int64_t threads = (int64_t)A.n * A.lanes;
   const int grid = (int)(stream ? ((int64_t)A.n + A.spmv_rb - 1) / A.spmv_rb : (threads + BLK - 1) / BLK);
-  auto go = [&](auto *kern) { hipLaunchKernelGGL(kern, dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y, stop); };
+  auto go = [&](auto *plain, auto *unless) {
+    if (stop) hipLaunchKernelGGL(unless, dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y, stop);
+    else hipLaunchKernelGGL(plain, dim3(grid), dim3(BLK), 0, s, A.n, A.rowptr, A.col, val, x, y);
+  };
   if (stream) {
     switch (A.spmv_rb) {
-      case 256: go(spmv_stream_kernel<T, 256, GUARD>); break;
-      case 128: go(spmv_stream_kernel<T, 128, GUARD>); break;
-      case 64: go(spmv_stream_kernel<T, 64, GUARD>); break;
-      default: go(spmv_stream_kernel<T, 32, GUARD>); break;
+      case 256: go(spmv_stream_kernel<T, 256>, spmv_stream_unless_kernel<T, 256>); break;
+      case 128: go(spmv_stream_kernel<T, 128>, spmv_stream_unless_kernel<T, 128>); break;
+      case 64: go(spmv_stream_kernel<T, 64>, spmv_stream_unless_kernel<T, 64>); break;
+      default: go(spmv_stream_kernel<T, 32>, spmv_stream_unless_kernel<T, 32>); break;
     }
   } else {
     switch (A.lanes) {
-      case 4: go(spmv_kernel<T, 4, GUARD>); break;
-      case 8: go(spmv_kernel<T, 8, GUARD>); break;
-      case 16: go(spmv_kernel<T, 16, GUARD>); break;
-      default: go(spmv_kernel<T, 32, GUARD>); break;
+      case 4: go(spmv_kernel<T, 4>, spmv_unless_kernel<T, 4>); break;
+      case 8: go(spmv_kernel<T, 8>, spmv_unless_kernel<T, 8>); break;
+      case 16: go(spmv_kernel<T, 16>, spmv_unless_kernel<T, 16>); break;
+      default: go(spmv_kernel<T, 32>, spmv_unless_kernel<T, 32>); break;
     }
   }
   SA_HIP(hipGetLastError());
@@ -231,14 +260,10 @@ int mat_norm_inf(const Mat &A, double *out) {
   return 0;
 }
 
-template <typename T>
-static int spmv_any(const Mat &A, const void *x, void *y, hipStream_t s, const int *stop) {
-  return stop ? spmv_t<T, true>(A, (const T *)x, (T *)y, stop, s) : spmv_t<T, false>(A, (const T *)x, (T *)y, stop, s);
-}
-
 int launch_spmv(const Mat &A, const void *x, void *y, hipStream_t s, const int *stop) {
   if (A.n == 0) return 0;
-  return A.prec == SA_FP64 ? spmv_any<double>(A, x, y, s, stop) : spmv_any<float>(A, x, y, s, stop);
+  if (A.prec == SA_FP64) return spmv_t<double>(A, (const double *)x, (double *)y, stop, s);
+  return spmv_t<float>(A, (const float *)x, (float *)y, stop, s);
 }
 
 // ---------------------------------------------------------------------------
